@@ -1,5 +1,5 @@
-// fp32 dense-layer GEMMs on CDNA4 matrix cores (the fp32 mode: PPO MLPs and
-// fp32 FlashSAC configurations; bf16 products run in gemm_bf16*.hip).
+// fp32 dense-layer GEMMs on the fp32 matrix instruction (mode 0), split-K reductions, transposes and the
+// rl_gemm entry point.
 //
 // One row-major kernel family covers the three products of a bias-free
 // Linear layer (the reference's CudaLinear plans, robolearn/cuda/linear.py:179-185):
@@ -17,17 +17,7 @@
 // staged through LDS in [row][k] order, 16 K per step, so each lane reads its
 // K-slice with two 16-byte LDS loads; the K order inside a step is permuted
 // identically for both operands, which leaves the dot products unchanged.
-//
-// Mode 2 runs the same products on the bf16 matrix cores at fp32 accuracy:
-// every operand value x is split exactly into three bf16 pieces
-// x = x0 + x1 + x2 (x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1),
-// each difference exact in fp32) when the tile is staged in LDS, and each 16-K
-// step issues six v_mfma_f32_32x32x16_bf16 for a0b0 + a0b1 + a1b0 + a0b2 + a1b1
-// + a2b0.  The pieces carry 3 x 8 significant bits and the three dropped
-// cross terms are below 2^-26 of the product, so a product is as accurate as
-// an fp32 one; the matrix-core time per 16-K step is 6 x 32 cycles instead of
-// 8 x 64 (v_mfma_f32_32x32x2_f32).  Staging, tiles and epilogues are shared
-// with mode 0.
+// Mode 2 (fp32 operands and results on the bf16 matrix cores) runs in gemm_split.hip.
 #include "gemm.hpp"
 
 #include <cmath>
@@ -36,27 +26,8 @@
 namespace rl {
 namespace gemm {
 
-constexpr int kFp32K = 32;              // K per LDS step: two 16-K MFMA substeps (16: 16.3 ms per c3 PPO update, 32: 15.4, 64: 21.1 -- occupancy 2)
+constexpr int kFp32K = 32;              // K per LDS step: two 16-K substeps
 constexpr int kFp32Pitch = kFp32K + 4;  // floats per LDS row
-constexpr int kSplitPitch = kFp32K + 8; // bf16 per LDS row of a split plane (80 bytes: row starts 20 banks apart)
-
-// x = x0 + x1 + x2 exactly in bf16 pieces, two values at a time: x0 keeps x's
-// top 8 significant bits (bf16 by truncation), r1 = x - x0 is exact in fp32
-// (same exponent), x1 keeps r1's top 8 bits, and r2 = r1 - x1 has at most 8
-// significant bits left, so x2 = r2 is exact in bf16.  Each piece's bf16 bits
-// are the high half of its fp32 bits; one byte permute packs the pieces of a
-// and b into a plane word (a in the low half).
-__device__ __forceinline__ void split3_pair(float a, float b, unsigned& p0, unsigned& p1, unsigned& p2) {
-    constexpr unsigned kHigh = 0xFFFF0000u;
-    constexpr unsigned kHighHalves = 0x07060302u;  // bytes 2, 3 of the second operand, then of the first
-    const unsigned ua = __float_as_uint(a), ub = __float_as_uint(b);
-    const float ra = a - __uint_as_float(ua & kHigh), rb = b - __uint_as_float(ub & kHigh);
-    const unsigned ura = __float_as_uint(ra), urb = __float_as_uint(rb);
-    const float sa = ra - __uint_as_float(ura & kHigh), sb = rb - __uint_as_float(urb & kHigh);
-    p0 = __builtin_amdgcn_perm(ub, ua, kHighHalves);
-    p1 = __builtin_amdgcn_perm(urb, ura, kHighHalves);
-    p2 = __builtin_amdgcn_perm(__float_as_uint(sb), __float_as_uint(sa), kHighHalves);
-}
 
 // Loads one Rows x kFp32K operand tile into registers (Threads threads) and
 // later stores it to LDS.  Element (r, k) of the operand is src[r * ld + k]
@@ -140,67 +111,17 @@ struct TileLoader {
             for (int e = 0; e < KPer; ++e) q[e] = regs[e];
         }
     }
-
-    // Mode 2: the three bf16 planes of the tile, plane p at lds + p * Rows * kSplitPitch.
-    __device__ __forceinline__ void store_split(unsigned short* lds) const {
-        constexpr int Plane = Rows * kSplitPitch;
-        const int t = threadIdx.x;
-        if constexpr (KContig) {
-#pragma unroll
-            for (int i = 0; i < PerThread; ++i) {
-                const int v = i * Threads + t;
-                const int offset = (v / VecPerRow) * kSplitPitch + (v % VecPerRow) * 4;
-                unsigned w[3][2];
-                split3_pair(regs[i * 4 + 0], regs[i * 4 + 1], w[0][0], w[1][0], w[2][0]);
-                split3_pair(regs[i * 4 + 2], regs[i * 4 + 3], w[0][1], w[1][1], w[2][1]);
-#pragma unroll
-                for (int q = 0; q < 3; ++q) *reinterpret_cast<uint2*>(lds + q * Plane + offset) = make_uint2(w[q][0], w[q][1]);
-            }
-        } else {
-            // KPer consecutive K values of one row: packed into 4-byte words per plane
-            static_assert(KPer % 2 == 0 && kSplitPitch % 2 == 0, "pairs of K values share a word");
-            const int offset = (t % Rows) * kSplitPitch + (t / Rows) * KPer;
-#pragma unroll
-            for (int e = 0; e < KPer; e += 2) {
-                unsigned w0, w1, w2;
-                split3_pair(regs[e], regs[e + 1], w0, w1, w2);
-                *reinterpret_cast<unsigned*>(lds + offset + e) = w0;
-                *reinterpret_cast<unsigned*>(lds + Plane + offset + e) = w1;
-                *reinterpret_cast<unsigned*>(lds + 2 * Plane + offset + e) = w2;
-            }
-        }
-    }
-
-    // Sum of this thread's staged values (row sums of an M-contiguous operand).
-    __device__ __forceinline__ float sum() const {
-        float total = 0.0f;
-#pragma unroll
-        for (int e = 0; e < Count; ++e) total += regs[e];
-        return total;
-    }
 };
 
-// NW waves own the T x T tile as WGM x WGN wave tiles of (T / WGM) x (T / WGN):
-// 4 waves as 2 x 2, 8 waves (mode 2, 128-wide tiles) as 2 x 4.
-// Eight-wave workgroups are held to 128 VGPRs, so that two of them (four waves per
-// SIMD) share a CU.
-template <int T, int NW, bool AK, bool BK, bool Split>
-__global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 4 : 1))) void gemm_kernel(
-    Params p) {
-    constexpr int Threads = NW * kWave;
-    constexpr int WGN = NW == 4 ? 2 : 4;
-    constexpr int WGM = NW / WGN;
+// Four waves own the T x T tile as 2 x 2 wave tiles of (T / 2) x (T / 2).
+template <int T, bool AK, bool BK>
+__global__ __launch_bounds__(kThreads) void gemm_kernel(Params p) {
+    constexpr int Threads = kThreads;
+    constexpr int WGN = 2, WGM = 2;
     constexpr int WTM = T / WGM, WTN = T / WGN;    // wave tile
     constexpr int WBM = WTM / 32, WBN = WTN / 32;  // 32x32 accumulator blocks per wave
-    static_assert((NW == 4 || NW == 8) && WBM >= 1 && WBN >= 1, "wave layouts");
-    constexpr int Plane = T * kSplitPitch;  // bf16 per split plane
-    constexpr int StageBytes = Split ? 3 * Plane * 2 : T * kFp32Pitch * 4;
-    __shared__ __attribute__((aligned(16))) unsigned char sa_raw[StageBytes];
-    __shared__ __attribute__((aligned(16))) unsigned char sb_raw[StageBytes];
-    float* sa = reinterpret_cast<float*>(sa_raw);
-    float* sb = reinterpret_cast<float*>(sb_raw);
-    unsigned short* ha = reinterpret_cast<unsigned short*>(sa_raw);
-    unsigned short* hb = reinterpret_cast<unsigned short*>(sb_raw);
+    __shared__ __attribute__((aligned(16))) float sa[T * kFp32Pitch];
+    __shared__ __attribute__((aligned(16))) float sb[T * kFp32Pitch];
 
     // XCD-aware tile order: workgroups are dispatched round-robin over the 8
     // XCDs in linear (x fastest) order, so logical tile id (w % 8) * (G / 8) +
@@ -256,21 +177,9 @@ __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(NW =
     };
 
     // B is indexed (n, k) when BK else (k, n); the loader wants (row=n, k).
-    // Mode 2 takes the row sums from the staged fp32 registers (M-contiguous A only).
     const auto stage = [&]() {
-        if constexpr (Split) {
-            la.store_split(ha);
-            lb.store_split(hb);
-            if constexpr (!AK) {
-                if (row_sums) {
-#pragma unroll
-                    for (int e = 0; e < decltype(la)::Count; ++e) add_sum(la.regs[e]);
-                }
-            }
-        } else {
-            la.store(sa);
-            lb.store(sb);
-        }
+        la.store(sa);
+        lb.store(sb);
     };
     // K steps whose operand tiles lie wholly inside A and B (uniform per workgroup) take the unchecked loads
     const bool a_full = (!AK || avec) && m0 + T <= p.m;
@@ -290,43 +199,6 @@ __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(NW =
     for (int k0 = k_begin; k0 < k_end; k0 += kFp32K) {
         const bool more = k0 + kFp32K < k_end;
         if (more) load_step(k0 + kFp32K);
-        if constexpr (Split) {
-#pragma unroll
-          for (int sub = 0; sub < kFp32K / 16; ++sub) {
-            bf16x8_t af[WBM][3], bf[WBN][3];
-            const int koff = 16 * sub + 8 * (lane / 32);
-#pragma unroll
-            for (int i = 0; i < WBM; ++i) {
-                const int off = (wm * WTM + i * 32 + lane % 32) * kSplitPitch + koff;
-#pragma unroll
-                for (int q = 0; q < 3; ++q) af[i][q] = *reinterpret_cast<const bf16x8_t*>(ha + q * Plane + off);
-            }
-#pragma unroll
-            for (int j = 0; j < WBN; ++j) {
-                const int off = (wn * WTN + j * 32 + lane % 32) * kSplitPitch + koff;
-#pragma unroll
-                for (int q = 0; q < 3; ++q) bf[j][q] = *reinterpret_cast<const bf16x8_t*>(hb + q * Plane + off);
-            }
-#pragma unroll
-            for (int i = 0; i < WBM; ++i) {
-#pragma unroll
-                for (int j = 0; j < WBN; ++j) {
-                    f32x16_t c = acc[i][j];
-                    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i][0], bf[j][0], c, 0, 0, 0);
-                    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i][0], bf[j][1], c, 0, 0, 0);
-                    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i][1], bf[j][0], c, 0, 0, 0);
-                    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i][0], bf[j][2], c, 0, 0, 0);
-                    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i][1], bf[j][1], c, 0, 0, 0);
-                    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i][2], bf[j][0], c, 0, 0, 0);
-                    acc[i][j] = c;
-                }
-            }
-          }
-            __syncthreads();
-            if (more) stage();
-            __syncthreads();
-            continue;
-        }
         if (row_sums) {
             const float* q = sa + (threadIdx.x / SumLanes) * kFp32Pitch + (threadIdx.x % SumLanes) * SumPer;
 #pragma unroll
@@ -365,22 +237,7 @@ __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(NW =
         __syncthreads();
     }
 
-    if (Split && !AK && row_sums) {
-        // thread t holds the partial sum of row t % T over its k group t / T: add the groups in order
-        float* part = sa;
-        part[threadIdx.x] = a_sum;
-        __syncthreads();
-        const int t = static_cast<int>(threadIdx.x);
-        if (t < T) {
-            float total = part[t];
-#pragma unroll
-            for (int g = 1; g < Threads / T; ++g) total += part[g * T + t];
-            const int r = m0 + t;
-            if (r < p.m)
-                p.a_sums[(p.splits == 1 ? batch * p.sums_stride
-                                         : (static_cast<long long>(split) * p.batch + batch) * p.m) + r] = total;
-        }
-    } else if (row_sums) {
+    if (row_sums) {
         // the SumLanes partial sums of a row sit in adjacent lanes: fixed-order butterfly
 #pragma unroll
         for (int offset = 1; offset < SumLanes; offset <<= 1) a_sum += __shfl_xor(a_sum, offset);
@@ -600,45 +457,29 @@ __global__ __launch_bounds__(256) void splitk_reduce_grouped(const float* work, 
     if (d_bf16) d_bf16[offset] = f32_to_bf16_bits(value);
 }
 
-// Workgroups of 128 x 128 tiles (all splits) from which a mode-2 product runs
-// them on eight waves: each split staged value then feeds twice the MFMAs of a
-// 64 x 64 tile, and the operand reads per product halve.  Outputs of at most 64
-// rows or columns (heads) keep the 64 x 64 tiles, which waste less of a tile.
-constexpr long long kSplitWideTiles = 256;
-
-// Output tile edge for an fp32 product: 64 unless 128-wide tiles would still
-// give every SIMD several waves of work (mode 0), or every CU a workgroup of
-// eight waves (mode 2).
-int fp32_tile(const Params& p, bool split) {
+// Output tile edge: 64 unless 128-wide tiles would still give every SIMD several waves of work.
+int fp32_tile(const Params& p) {
     const long long big = static_cast<long long>(ceil_div(p.m, 128)) * ceil_div(p.n, 128) * p.batch * p.splits;
-    if (split) return p.m > 64 && p.n > 64 && big >= kSplitWideTiles ? 128 : 64;
     return big >= 2048 ? 128 : 64;
 }
 
-template <int T, int NW, bool AK, bool BK, bool Split>
+template <int T, bool AK, bool BK>
 void launch_fp32_tiled(const Params& p, hipStream_t stream) {
     const dim3 grid(ceil_div(p.n, T), ceil_div(p.m, T), static_cast<unsigned>(p.batch * p.splits));
-    hipLaunchKernelGGL((gemm_kernel<T, NW, AK, BK, Split>), grid, dim3(NW * kWave), 0, stream, p);
+    hipLaunchKernelGGL((gemm_kernel<T, AK, BK>), grid, dim3(kThreads), 0, stream, p);
 }
 
-template <bool AK, bool BK, bool Split>
+template <bool AK, bool BK>
 void launch_fp32_layout(const Params& p, hipStream_t stream) {
-    if (fp32_tile(p, Split) == 128) launch_fp32_tiled<128, Split ? 8 : 4, AK, BK, Split>(p, stream);
-    else launch_fp32_tiled<64, 4, AK, BK, Split>(p, stream);
+    if (fp32_tile(p) == 128) launch_fp32_tiled<128, AK, BK>(p, stream);
+    else launch_fp32_tiled<64, AK, BK>(p, stream);
 }
 
-template <bool Split>
-void launch_fp32_mode(const Params& p, bool ak, bool bk, hipStream_t stream) {
-    if (ak && bk) launch_fp32_layout<true, true, Split>(p, stream);
-    else if (ak && !bk) launch_fp32_layout<true, false, Split>(p, stream);
-    else if (!ak && bk) launch_fp32_layout<false, true, Split>(p, stream);
-    else launch_fp32_layout<false, false, Split>(p, stream);
-}
-
-// split: mode 2 (three-piece bf16 products); row sums of a K-contiguous A stay on mode 0
-void launch_fp32(const Params& p, bool ak, bool bk, bool split, hipStream_t stream) {
-    if (split && !(p.a_sums && ak)) launch_fp32_mode<true>(p, ak, bk, stream);
-    else launch_fp32_mode<false>(p, ak, bk, stream);
+void launch_fp32(const Params& p, bool ak, bool bk, hipStream_t stream) {
+    if (ak && bk) launch_fp32_layout<true, true>(p, stream);
+    else if (ak && !bk) launch_fp32_layout<true, false>(p, stream);
+    else if (!ak && bk) launch_fp32_layout<false, true>(p, stream);
+    else launch_fp32_layout<false, false>(p, stream);
 }
 
 // dst[b][c][r] = src[b][r][c] for 16-bit elements: 64 x 64 tiles through LDS,
@@ -838,7 +679,9 @@ int run_gemm(int mode, int a_bf16, int b_bf16, int a_kcontig, int b_kcontig, int
     p.moments = fused_moments ? moments : nullptr;
     if (mode == 1) gemm::launch_bf16(p, a_bf16, b_bf16, a_kcontig != 0, b_kcontig != 0, stream);
     else if (mode == 3) gemm::launch_f16(p, a_bf16, b_bf16, a_kcontig != 0, b_kcontig != 0, stream);
-    else gemm::launch_fp32(p, a_kcontig != 0, b_kcontig != 0, mode == 2, stream);
+    else if (mode == 2 && gemm::split_eligible(p, a_kcontig != 0, b_kcontig != 0))
+        gemm::launch_split(p, a_kcontig != 0, b_kcontig != 0, stream);
+    else gemm::launch_fp32(p, a_kcontig != 0, b_kcontig != 0, stream);
     check_launch("Launch GEMM");
     if (splits > 1) {
         const long long total = static_cast<long long>(batch) * m * n;

@@ -57,6 +57,10 @@ __device__ __forceinline__ float apply_epilogue(float v, int epilogue) {
     return v;
 }
 
+// fp32 products from three bf16 pieces per operand value (gemm_split.hip); split_eligible: the layouts it takes.
+bool split_eligible(const Params& p, bool ak, bool bk);
+void launch_split(const Params& p, bool ak, bool bk, hipStream_t stream);
+
 // bf16 MFMA kernel family with 256x128 tiles (gemm_bf16.hip).
 void launch_bf16(const Params& p, int a_bf16, int b_bf16, bool ak, bool bk, hipStream_t stream);
 // The same tiles on IEEE fp16 operands (a_f16 / b_f16: 16-bit fp16 storage,

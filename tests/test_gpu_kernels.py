@@ -653,3 +653,55 @@ def test_fp32_split_products_are_fp32_accurate(gpu, batch, rows, out_dim, in_dim
         err_split = (split[key] - ref).abs().max().item()
         assert err_split <= 4.0 * err_native + 2e-7 * scale, (key, err_split, err_native, scale)
         assert err_split <= 2e-6 * scale * max(1.0, math.sqrt(length[key] / 2048)), (key, err_split, scale)
+
+
+# rows and columns at the edges of the 64- and 128-wide tiles, K at the edges of the 32-deep steps; the last two
+# run the 128-wide tiles
+RANGE_SHAPES = [(1, 1, 1, 1), (63, 65, 31, 1), (64, 64, 32, 1), (129, 70, 33, 3), (130, 64, 200, 4),
+                 (2100, 2050, 97, 1), (300, 390, 3000, 32)]
+
+
+@pytest.mark.parametrize("a_kcontig,b_kcontig", [(True, True), (True, False), (False, True), (False, False)])
+@pytest.mark.parametrize("m,n,k,splits", RANGE_SHAPES)
+def test_fp32_split_products_over_the_exponent_range(gpu, m, n, k, splits, a_kcontig, b_kcontig):
+    """Mode 2 over rows of magnitudes 1e-30 to 1e12, rows that are zero, start with zeros or grow by 1e6 along
+    K, and rows that hold an infinity or a NaN, which must reach no other row or column.
+
+    Bound per element: each of the 6 ceil(k / 16) accumulations, like each of the partial sums, rounds once at
+    2^-23 (the matrix instruction may truncate) of sums that Cauchy-Schwarz bounds by the row's times the
+    column's norm; the dropped products are below 2^-26 each."""
+    print(f"case split range m={m} n={n} k={k} splits={splits} ak={a_kcontig} bk={b_kcontig}", flush=True)
+    g = torch.Generator().manual_seed(m + 3 * n + 7 * k)
+    a, b = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g)
+    a *= 10.0 ** (torch.arange(m) % 43 - 30.0)[:, None]
+    b *= 10.0 ** (torch.arange(n) % 29 - 14.0)[:, None]
+    grow = torch.arange(k) >= k // 2
+    a[2::11, grow] *= 1e6
+    b[3::13, grow] *= 1e6
+    a[4::11, : k // 2] = 0.0
+    a[5::17] = 0.0
+    bad_a, bad_b = (m // 2, n // 3) if min(m, n) > 1 else (m, n)  # the rows with non-finite values
+    if bad_a < m:
+        a[bad_a, k // 2], b[bad_b, k - 1] = float("inf"), float("nan")
+    ad, bd = (t.to(gpu).contiguous() for t in (a if a_kcontig else a.t(), b if b_kcontig else b.t()))
+    d = torch.full((m, n), 7.0, device=gpu)
+    sums = torch.full((m,), 7.0, device=gpu) if not a_kcontig else None
+    workspace = torch.empty(splits * (m * n + m) * 4, dtype=torch.uint8, device=gpu) if splits > 1 else None
+    K.gemm(ad, bd, d, m=m, n=n, k=k, a_kcontig=a_kcontig, b_kcontig=b_kcontig, lda=k if a_kcontig else m,
+           ldb=k if b_kcontig else n, ldd=n, mode=K.FP32_SPLIT, splits=splits, workspace=workspace, a_sums=sums)
+    got = d.cpu().double()
+    if bad_a < m:
+        assert not torch.isfinite(got[bad_a]).any() and not torch.isfinite(got[:, bad_b]).any()
+    rows, cols = torch.arange(m) != bad_a, torch.arange(n) != bad_b
+    a64, b64 = a.double()[rows], b.double()[cols]
+    expected = a64 @ b64.t()
+    norms = a64.norm(dim=1)[:, None] * b64.norm(dim=1)[None, :]
+    bound = norms * (4 + 2 * 6 * math.ceil(k / 16) + 2 * splits) * 2.0**-24 + 2.0**-126
+    # products past fp32's range: infinite on both sides, or not compared
+    finite = norms < 1e38
+    error = (got[rows][:, cols] - expected).abs()
+    assert (error <= bound)[finite].all(), float((error / bound)[finite].max())
+    if sums is not None:
+        total = a64.sum(1)
+        slack = a64.abs().sum(1) * (8 + splits) * 2.0**-23
+        assert ((sums.cpu().double()[rows] - total).abs() <= slack).all()
