@@ -164,7 +164,7 @@ def last_error() -> str:
 
 def call(name: str, *args) -> int:
     """Call a status-returning entry point and raise on -1."""
-    result = getattr(load(), name)(*args)
+    result = getattr(_LIBRARY or load(), name)(*args)
     if result != 0:
         raise RuntimeError(f"{name}: {last_error()}")
     return result

@@ -92,6 +92,9 @@ class WarpPPO:
             self.names = [n for n, _ in actor] + [n for n, _ in critic] + ["std"]
             views = self.flat.params()
             self.parameters = [views[n] for n in self.names]
+            # (weight, bias) views per layer: building them anew costs the host about 1 us a view and call
+            self._layers = {(prefix, i): (views[f"{prefix}.{i}.weight"], views[f"{prefix}.{i}.bias"])
+                            for prefix in ("actor", "critic") for i in range(self.layers)}
             self.grads = self.flat.grads()
             rng = np.random.default_rng(cfg.seed)
             for n, shape in actor + critic:
@@ -192,8 +195,7 @@ class WarpPPO:
 
     # ------------------------------------------------------------------
     def _layer(self, prefix, i):
-        p = self.flat.params()
-        return p[f"{prefix}.{i}.weight"], p[f"{prefix}.{i}.bias"]
+        return self._layers[prefix, i]
 
     def _mlp_forward(self, prefix, x, rows, hidden, out, x_ld=None):
         """Linear + ELU hidden layers (ELU fused in the GEMM epilogue), linear output.
@@ -208,30 +210,32 @@ class WarpPPO:
         w, b = self._layer(prefix, self.layers - 1)
         K.linear_forward(inputs, w, out, rows=rows, in_dim=widths[-1], out_dim=out.shape[1], bias=b, mode=self.gemm_mode)
 
-    def _joint_forward(self, rows):
-        """Both MLPs on the minibatch observations: each hidden layer is one batch-2 product over
+    def _joint_forward(self, rows, x, x_ld, h_pair, head_out):
+        """Both MLPs on `rows` rows of x (row pitch x_ld): each hidden layer is one batch-2 product over
         the actor and critic weights (Linear + bias + ELU in the GEMM epilogue), then the two
-        output layers (mean, value)."""
+        output layers (mean, value) as one batch-2 product."""
         hidden = self.config.hidden_dims
         widths = (self.observation_dim, *hidden)
         for i, width in enumerate(hidden):
             w, b = self._layer("actor", i)
             first = i == 0
-            K.gemm(self.b_obs if first else self.h_pair[i - 1], w, self.h_pair[i], m=rows, n=width, k=widths[i],
-                   batch=2, a_kcontig=True, b_kcontig=True, lda=self.obs_ld if first else widths[i], ldb=widths[i],
+            K.gemm(x if first else h_pair[i - 1], w, h_pair[i], m=rows, n=width, k=widths[i],
+                   batch=2, a_kcontig=True, b_kcontig=True, lda=x_ld if first else widths[i], ldb=widths[i],
                    ldd=width, stride_a=0 if first else rows * widths[i], stride_b=self.w_stride[i],
                    stride_d=rows * width, bias=b, stride_bias=self.b_stride[i], epilogue="elu", mode=self.gemm_mode)
-        last = self.layers - 1
+        w, b = self._layer("actor", self.layers - 1)
+        A, width = self.action_dim, widths[-1]
+        K.gemm(h_pair[-1], w, head_out, m=rows, n=A, k=width, batch=2, a_kcontig=True, b_kcontig=True,
+               lda=width, ldb=width, ldd=A, stride_a=rows * width, stride_b=self.head_w_stride,
+               stride_d=rows * A, bias=b, stride_bias=self.head_b_stride, mode=self.gemm_mode)
+
+    def _minibatch_forward(self, rows):
         if self.batched_heads:
-            w, b = self._layer("actor", last)
-            A, width = self.action_dim, widths[-1]
-            K.gemm(self.h_pair[-1], w, self.head_out, m=rows, n=A, k=width, batch=2, a_kcontig=True, b_kcontig=True,
-                   lda=width, ldb=width, ldd=A, stride_a=rows * width, stride_b=self.head_w_stride,
-                   stride_d=rows * A, bias=b, stride_bias=self.head_b_stride, mode=self.gemm_mode)
+            self._joint_forward(rows, self.b_obs, self.obs_ld, self.h_pair, self.head_out)
             return
-        for member, (prefix, out) in enumerate((("actor", self.mean), ("critic", self.value))):
-            w, b = self._layer(prefix, last)
-            K.linear_forward(self.b_obs, w, out, rows=rows, in_dim=widths[-1], out_dim=out.shape[1], bias=b,
+        for prefix, out in (("actor", self.mean), ("critic", self.value)):  # no hidden layers
+            w, b = self._layer(prefix, 0)
+            K.linear_forward(self.b_obs, w, out, rows=rows, in_dim=self.observation_dim, out_dim=out.shape[1], bias=b,
                              mode=self.gemm_mode, x_ld=self.obs_ld)
 
     def _joint_backward(self, rows):
@@ -304,7 +308,7 @@ class WarpPPO:
                      self.stds.data_ptr(), self.b_obs.data_ptr(), self.b_actions.data_ptr(),
                      self.b_log_probs.data_ptr(), self.b_values.data_ptr(), self.b_advantages.data_ptr(),
                      self.b_returns.data_ptr(), self.b_means.data_ptr(), self.b_stds.data_ptr(), K.stream())
-        self._joint_forward(M)
+        self._minibatch_forward(M)
         # loss, its gradients, the pre-step KL with the adaptive learning rate and the std-parameter
         # gradient: two launches (ppo.py:207-310)
         _native.call("rl_ppo_minibatch_loss", self.mean.data_ptr(), A, self.value.data_ptr(), self.value_ld,
@@ -371,9 +375,17 @@ class WarpPPO:
         if n not in self._act_buffers:
             z = lambda *s: torch.zeros(*s, device=self.device)  # noqa: E731
             A = self.action_dim
-            self._act_buffers[n] = dict(hidden=[z(n, w) for w in self.config.hidden_dims], mean=z(n, A),
-                                        value=z(n, 1), noise=z(n, A), actions=z(n, A), log_probs=z(n), values=z(n),
-                                        std=z(A), next_value=z(n, 1))
+            # hidden activations as actor/critic pairs and, with hidden layers, [2, n, A] head outputs: member 0
+            # the mean, column 0 of member 1 the value (the layout of the update's batched forward)
+            b = dict(hidden=[z(2, n, w) for w in self.config.hidden_dims], noise=z(n, A), actions=z(n, A),
+                     log_probs=z(n), values=z(n), std=z(A), next_value=z(n, 1))
+            if self.batched_heads:
+                b["head"] = z(2, n, A)
+                b["mean"], b["value"], b["value_ld"] = b["head"][0], b["head"][1][:, :1], A
+            else:
+                b["mean"], b["value"], b["value_ld"] = z(n, A), z(n, 1), 1
+            b["critic_hidden"] = [h[1] for h in b["hidden"]]
+            self._act_buffers[n] = b
         return self._act_buffers[n]
 
     @torch.no_grad()
@@ -391,13 +403,16 @@ class WarpPPO:
         b = self._act_state(n)
         cfg = self.config
         with torch.cuda.device(self.device):
-            self._mlp_forward("actor", obs, n, b["hidden"], b["mean"])
-            self._mlp_forward("critic", obs, n, b["hidden"], b["value"])
+            if self.batched_heads:
+                self._joint_forward(n, obs, self.observation_dim, b["hidden"], b["head"])
+            else:
+                self._mlp_forward("actor", obs, n, [], b["mean"])
+                self._mlp_forward("critic", obs, n, [], b["value"])
             noise = None
             if not deterministic:
                 K.philox_normal(b["noise"], seed=cfg.seed * 7919 + 53, counter=self._act_counter, stream_id=53)
                 noise = b["noise"]
-            _native.call("rl_ppo_sample", b["mean"].data_ptr(), self.action_dim, b["value"].data_ptr(), 1,
+            _native.call("rl_ppo_sample", b["mean"].data_ptr(), self.action_dim, b["value"].data_ptr(), b["value_ld"],
                          self.distribution_parameter.data_ptr(), int(cfg.std_type == "scalar"),
                          float(cfg.std_range[0]), float(cfg.std_range[1]),
                          noise.data_ptr() if noise is not None else None, n, self.action_dim,
@@ -423,7 +438,7 @@ class WarpPPO:
         truncated = torch.as_tensor(truncated, device=dev).reshape(n).to(torch.int32).contiguous()
         obs, next_obs = obs.contiguous(), next_obs.contiguous()
         with torch.cuda.device(dev):
-            self._mlp_forward("critic", next_obs, n, b["hidden"], b["next_value"])
+            self._mlp_forward("critic", next_obs, n, b["critic_hidden"], b["next_value"])
             _native.call("rl_ppo_store", int(step), n, self.observation_dim, self.action_dim, obs.data_ptr(),
                          b["actions"].data_ptr(), b["log_probs"].data_ptr(), b["values"].data_ptr(),
                          rewards.data_ptr(), terminated.data_ptr(), truncated.data_ptr(), b["next_value"].data_ptr(),

@@ -449,3 +449,32 @@ def test_update_with_wide_observations_matches_oracle(gpu):
     assert health["value_loss"] == pytest.approx(result["value_loss"], rel=1e-4, abs=1e-6)
     for i, p in enumerate(oracle.params):
         np.testing.assert_allclose(state[f"parameter_{i}"], p.detach().numpy(), atol=2e-4, rtol=0, err_msg=str(i))
+
+
+@pytest.mark.parametrize("hidden", [(), (32,), (512, 256, 128)])
+@pytest.mark.parametrize("rows", [1, 65, 300])
+def test_rollout_forward_matches_float64(gpu, hidden, rows):
+    """act() and store() against float64 MLPs: no hidden layer (two separate products), one, and the batched
+    actor/critic forward; 1e-5 covers three layers of fp32 sums of at most 512 terms."""
+    print(f"case rollout forward hidden={hidden} rows={rows}", flush=True)
+    from robolearn_amd.ppo import WarpPPO
+
+    agent = WarpPPO(11, 3, rows, 1, PPOConfig(hidden_dims=hidden, activation="elu"))
+    g = torch.Generator().manual_seed(rows)
+    obs, following = torch.randn(rows, 11, generator=g), torch.randn(rows, 11, generator=g)
+    agent.act(obs.to(gpu))
+    zeros = torch.zeros(rows, dtype=torch.int32, device=gpu)
+    agent.store(0, obs.to(gpu), torch.zeros(rows, device=gpu), zeros, zeros, following.to(gpu))
+    weights = [p.detach().cpu().double() for p in agent.parameters]
+    layers = len(hidden) + 1
+
+    def mlp(x, first):
+        for i in range(layers):
+            x = x @ weights[first + 2 * i].t() + weights[first + 2 * i + 1]
+            if i + 1 < layers:
+                x = torch.nn.functional.elu(x)
+        return x
+
+    for got, x, first in ((agent.means, obs, 0), (agent.values[:, None], obs, 2 * layers),
+                          (agent.next_values[:, None], following, 2 * layers)):
+        torch.testing.assert_close(got.cpu().double(), mlp(x.double(), first), rtol=1e-5, atol=1e-5)
