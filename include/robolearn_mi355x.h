@@ -323,6 +323,19 @@ int rl_scale_rewards(float* rewards, long long n, const float* var, const float*
 int rl_exploration_noise(unsigned long long seed, long long* step, const float* cdf, int max_n, int* state,
                          float* cached_noise, long long count, const float* uniform, const float* fresh_noise,
                          void* stream);
+/* Actions of the eval-mode actor for `rows` observations (row pitch ld_obs) in one
+ * launch: input BatchNorm, embedder, `blocks` residual blocks, RMSNorm, heads, and
+ * tanh(mean) (noise NULL) or tanh(mean + std * noise), noise [rows, action_dim].
+ * parameters: host array of 8 + 10 * blocks device pointers, read at the call:
+ * input norm (running mean, running variance, weight, bias), embedder [hidden, obs_dim],
+ * per block W1 [4 hidden, hidden] and its norm (four pointers), W2 [hidden, 4 hidden] and
+ * its norm, then the post-norm weight, the mean and log-std head rows [2 action_dim,
+ * hidden] and their bias [2 action_dim].  hidden and 2 * action_dim up to 256, obs_dim up
+ * to 1024 (512 with hidden <= 128), blocks up to 8.  Replaces the act path of
+ * robolearn/flashsac/agent.py:414-455 (networks.py:37-61, layers.py:67-166). */
+int rl_actor_act(long long rows, int obs_dim, int hidden, int blocks, int action_dim, const float* obs,
+                 long long ld_obs, const void* const* parameters, const float* noise, float* actions, float bn_eps,
+                 float rms_eps, void* stream);
 /* Replay ingest of one vector step (replaces TorchUniformBuffer.add,
  * robolearn/flashsac/replay.py:107-174, and the Warp staging kernels
  * _copy_pending/_commit_pending/_advance_replay, robolearn/warp/_flash_replay.py:26-113).

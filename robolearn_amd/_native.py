@@ -115,6 +115,7 @@ SIGNATURES = {
     "rl_replay_ingest": (c_int, [c_ll, c_int, c_int, c_int, c_ll, c_float] + [P] * 6 + [P] * 4 + [P] * 7
                          + [P, P]),
     "rl_reward_stats_update": (c_int, [c_ll, c_float, P, P, P, P, P, P, P]),
+    "rl_actor_act": (c_int, [c_ll, c_int, c_int, c_int, c_int, P, c_ll, PP, P, P, c_float, c_float, P]),
     # PPO
     "rl_gae": (c_int, [c_int, c_int, c_float, c_float, c_int, P, P, P, P, P, P, P, P]),
     "rl_normalize_advantages": (c_int, [P, c_ll, c_int, P, P]),

@@ -281,6 +281,7 @@ class FlashSAC:
             self.exploration_step = torch.zeros(1, dtype=torch.long, device=dev)
             self.exploration_noise = torch.zeros(num_envs, action_dim, device=dev)
             self._act_nets = {}
+            self._act_parameters = self._actor_pointers()
         self.metrics = {key: self.metrics_buffer[i: i + 1] for i, key in enumerate(METRIC_KEYS)}
 
     # ------------------------------------------------------------------
@@ -595,6 +596,18 @@ class FlashSAC:
             self._act_nets[n] = (net, head, actions)
         return self._act_nets[n]
 
+    def _actor_pointers(self):
+        """The fp32 actor's tensors in rl_actor_act's order."""
+        p, running = self.actor_p, self.actor_running
+        norm = lambda name: [running[name + ".running_mean"], running[name + ".running_var"],  # noqa: E731
+                             p[name + ".weight"], p[name + ".bias"]]
+        tensors = norm("embedder.norm") + [p["embedder.w.w.weight"]]
+        for i in range(self.cfg.actor_num_blocks):
+            for j in (1, 2):
+                tensors += [p[f"encoder.{i}.w{j}.w.weight"]] + norm(f"encoder.{i}.norm{j}")
+        tensors += [p["post_norm.weight"], self.head_w, self.head_b]
+        return _native.pointer_array([t.data_ptr() for t in tensors])
+
     @torch.no_grad()
     def act(self, observations: torch.Tensor, training: bool = True) -> torch.Tensor:
         """Normalized actions from the eval-mode actor (agent.py:583-585 -> sample_actions :414-455).
@@ -606,18 +619,11 @@ class FlashSAC:
         obs = torch.as_tensor(observations, device=self.device, dtype=torch.float32)
         if obs.dim() != 2 or obs.shape[1] < self.observation_dim:
             raise ValueError("act() expects [rows, obs] observations with the actor's observation prefix.")
-        obs = obs[:, : self.observation_dim].contiguous()
         n = obs.shape[0]
         if training and n != self.num_envs:
             raise ValueError("Training action batches must match num_envs.")
-        A = self.action_dim
-        net, head, actions = self._act_net(n)
-        p = self.actor_p
+        A, p = self.action_dim, self.actor_p
         with torch.cuda.device(self.device):
-            net.forward(p, p, self.actor_running, obs, rows=n, x_stride=0, training=False)
-            net.post_norm(p, rows=n, row0=0, count=n)
-            K.linear_forward(net.z, self.head_w, head, rows=n, in_dim=net.h, out_dim=2 * A, bias=self.head_b,
-                             mode=K.FP32_SPLIT)
             noise = None
             if training:
                 _native.call("rl_exploration_noise", self.cfg.seed * 7919 + 37, self.exploration_step.data_ptr(),
@@ -625,6 +631,19 @@ class FlashSAC:
                              self.exploration_state.data_ptr(), self.exploration_noise.data_ptr(), n * A, None, None,
                              K.stream())
                 noise = self.exploration_noise
+            if K.actor_act_fits(n, self.observation_dim, self.cfg.actor_hidden_dim, self.cfg.actor_num_blocks, A):
+                if obs.stride(1) != 1 or obs.stride(0) < self.observation_dim:
+                    obs = obs[:, : self.observation_dim].contiguous()
+                actions = torch.empty(n, A, device=self.device)
+                K.actor_act(obs, self._act_parameters, noise, actions, obs_dim=self.observation_dim,
+                            hidden=self.cfg.actor_hidden_dim, blocks=self.cfg.actor_num_blocks, action_dim=A)
+                return actions
+            obs = obs[:, : self.observation_dim].contiguous()
+            net, head, actions = self._act_net(n)
+            net.forward(p, p, self.actor_running, obs, rows=n, x_stride=0, training=False)
+            net.post_norm(p, rows=n, row0=0, count=n)
+            K.linear_forward(net.z, self.head_w, head, rows=n, in_dim=net.h, out_dim=2 * A, bias=self.head_b,
+                             mode=K.FP32_SPLIT)
             K.tanh_gaussian_forward(head, noise, actions, None, rows=n, action_dim=A, deterministic=not training)
             return actions.clone()
 
