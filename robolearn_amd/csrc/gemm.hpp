@@ -67,6 +67,10 @@ void launch_bf16(const Params& p, int a_bf16, int b_bf16, bool ak, bool bk, hipS
 // else fp32 rounded to fp16 on load).
 void launch_f16(const Params& p, int a_f16, int b_f16, bool ak, bool bk, hipStream_t stream);
 
+// 64x64-tile bf16 kernel for narrow or small products (gemm_bf16_narrow.hip).
+bool narrow_eligible(const Params& p, int a_bf16, int b_bf16);
+void launch_narrow(const Params& p, bool ak, bool bk, hipStream_t stream);
+
 // 256x256-tile bf16 kernel for exactly tiling bf16 operands (gemm_bf16_big.hip).
 bool big_eligible(const Params& p, int a_bf16, int b_bf16);
 void launch_big(const Params& p, bool ak, bool bk, hipStream_t stream);

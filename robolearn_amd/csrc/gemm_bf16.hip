@@ -376,6 +376,10 @@ void launch_bf16(const Params& p, int a_bf16, int b_bf16, bool ak, bool bk, hipS
         launch_big(p, ak, bk, stream);
         return;
     }
+    if (narrow_eligible(p, a_bf16, b_bf16)) {
+        launch_narrow(p, ak, bk, stream);
+        return;
+    }
     using F = float;
     using H = unsigned short;
     if (!a_bf16 && !b_bf16) launch_layout_v2<F, F>(p, ak, bk, stream);
