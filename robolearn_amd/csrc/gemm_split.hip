@@ -18,8 +18,6 @@
 // us, and 4096 x 256 x 1024 (one member) 30.7 -> 20.1 us.  Not kept: 64 x 64 wave tiles and a second LDS buffer
 // (one barrier per step), slower at two and three waves per SIMD; two fp16 pieces under per-row exponents (three
 // products), a further 10-20 % faster but not the same rounding.
-#include <algorithm>
-
 #include "gemm.hpp"
 
 namespace rl {
@@ -65,12 +63,12 @@ struct SplitLoader {
     int k_first;             // M/N-contiguous: first K of this thread
 
     __device__ __forceinline__ int row(int i) const {
-        const int t = static_cast<int>(threadIdx.x) % Threads;
+        const int t = static_cast<int>(threadIdx.x);
         return KContig ? t / Vec + i * (Threads / Vec) : t % Rows;
     }
 
     __device__ __forceinline__ void init(long long ld, int rows) {
-        const int t = static_cast<int>(threadIdx.x) % Threads;
+        const int t = static_cast<int>(threadIdx.x);
 #pragma unroll
         for (int i = 0; i < Owned; ++i) {
             const unsigned r = static_cast<unsigned>(min(row(i), rows - 1));
@@ -150,22 +148,15 @@ struct SplitLoader {
 
 // TM x TN output tile of WGM x WGN waves; MinWaves: the waves per SIMD the register allocation aims at (the 128
 // x 128 kernels fit 128 registers, so four waves, under a bound of 2 too, with better schedules: 99.4 -> 96.3 us).
-//
-// KGroups > 1: the workgroup is KGroups such sets of waves on one output tile.  Set g takes K steps g, g + KGroups,
-// ... through LDS tiles of its own, and set 0 adds the other sets' sums in order before its epilogue.
-template <int TM, int TN, int WGM, int WGN, int Step, int MinWaves, int KGroups, bool AK, bool BK>
-__global__ __launch_bounds__(WGM * WGN * kWave * KGroups) __attribute__((amdgpu_waves_per_eu(MinWaves))) void split_kernel(
+template <int TM, int TN, int WGM, int WGN, int Step, int MinWaves, bool AK, bool BK>
+__global__ __launch_bounds__(WGM * WGN * kWave) __attribute__((amdgpu_waves_per_eu(MinWaves))) void split_kernel(
     Params p) {
-    constexpr int Threads = WGM * WGN * kWave;  // of one set
+    constexpr int Threads = WGM * WGN * kWave;
     constexpr int WTM = TM / WGM, WTN = TN / WGN;  // wave tile
     constexpr int WBM = WTM / 32, WBN = WTN / 32;  // 32x32 accumulator blocks per wave
     constexpr int PlaneA = TM * Step, PlaneB = TN * Step;
-    __shared__ __attribute__((aligned(16))) unsigned short staged_a[KGroups * 3 * PlaneA];
-    __shared__ __attribute__((aligned(16))) unsigned short staged_b[KGroups * 3 * PlaneB];
-    // uniform over a wave
-    const int group = KGroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / Threads);
-    unsigned short* const sa = staged_a + group * 3 * PlaneA;
-    unsigned short* const sb = staged_b + group * 3 * PlaneB;
+    __shared__ __attribute__((aligned(16))) unsigned short sa[3 * PlaneA];
+    __shared__ __attribute__((aligned(16))) unsigned short sb[3 * PlaneB];
 
     // XCD-aware tile order: workgroups are dispatched round-robin over the 8 XCDs in linear (x fastest) order,
     // so logical tile id (w % 8) * (G / 8) + w / 8 gives each XCD a contiguous range of tiles; the N tiles of
@@ -186,7 +177,7 @@ __global__ __launch_bounds__(WGM * WGN * kWave * KGroups) __attribute__((amdgpu_
     const float* B = static_cast<const float*>(p.b) + batch * p.stride_b + (BK ? n0 * p.ldb + k_begin : k_begin * p.ldb + n0);
     const long long step_a = AK ? Step : Step * p.lda, step_b = BK ? Step : Step * p.ldb;
 
-    const int t = static_cast<int>(threadIdx.x) % Threads;
+    const int t = static_cast<int>(threadIdx.x);
     const int lane = t % kWave, wave = t / kWave;
     const int wm = wave / WGN, wn = wave % WGN;
 
@@ -206,7 +197,7 @@ __global__ __launch_bounds__(WGM * WGN * kWave * KGroups) __attribute__((amdgpu_
     // Row sums of op(A) over this split's K (the bias gradient of a weight-gradient product), by the workgroups
     // of the first N tile, from the staged fp32 values.  Compensated (Kahan) sums per group of 8 K: bias
     // gradients add thousands of values that largely cancel, where plain fp32 sums lose digits.
-    const bool row_sums = KGroups == 1 && !AK && p.a_sums != nullptr && bx == 0;
+    const bool row_sums = !AK && p.a_sums != nullptr && bx == 0;
     constexpr int SumGroups = AK ? 1 : decltype(la)::Count / 8;
     float a_sum[SumGroups] = {}, a_comp[SumGroups] = {};
     const auto add_sums = [&]() {
@@ -259,94 +250,38 @@ __global__ __launch_bounds__(WGM * WGN * kWave * KGroups) __attribute__((amdgpu_
         la.store(sa);
         lb.store(sb);
         add_sums();
-        A += KGroups * step_a;
-        B += KGroups * step_b;
+        A += step_a;
+        B += step_b;
     };
 
     const int full = k_count / Step, tail = k_count % Step;
-    if constexpr (KGroups == 1) {
-        if (full > 0) {
-            la.load(A, p.lda);
-            lb.load(B, p.ldb);
-        } else {
-            la.load_tail(A, p.lda, tail);
-            lb.load_tail(B, p.ldb, tail);
-        }
-        stage();
-        // one step in LDS, the next on its way to registers; only the last load can be short
-        for (int s = 1; s < full; ++s) {
-            la.load(A, p.lda);
-            lb.load(B, p.ldb);
-            __syncthreads();
-            multiply();
-            __syncthreads();
-            stage();
-        }
-        if (full > 0 && tail > 0) {
-            la.load_tail(A, p.lda, tail);
-            lb.load_tail(B, p.ldb, tail);
-            __syncthreads();
-            multiply();
-            __syncthreads();
-            stage();
-        }
+    if (full > 0) {
+        la.load(A, p.lda);
+        lb.load(B, p.ldb);
+    } else {
+        la.load_tail(A, p.lda, tail);
+        lb.load_tail(B, p.ldb, tail);
+    }
+    stage();
+    // one step in LDS, the next on its way to registers; only the last load can be short
+    for (int s = 1; s < full; ++s) {
+        la.load(A, p.lda);
+        lb.load(B, p.ldb);
         __syncthreads();
         multiply();
-    } else {
-        // every set passes the same barriers: a set that has run out of steps skips only its loads and products
-        const int steps = full + (tail > 0);
-        const auto load = [&](int s) {
-            if (s < full) {
-                la.load(A, p.lda);
-                lb.load(B, p.ldb);
-            } else if (s < steps) {
-                la.load_tail(A, p.lda, tail);
-                lb.load_tail(B, p.ldb, tail);
-            }
-        };
-        A += group * step_a;
-        B += group * step_b;
-        int s = group;  // the step in LDS
-        load(s);
-        if (s < steps) stage();
-        for (int first = KGroups; first < steps; first += KGroups) {
-            load(s + KGroups);
-            __syncthreads();
-            multiply();
-            __syncthreads();
-            s += KGroups;
-            if (s < steps) stage();
-        }
         __syncthreads();
-        if (s < steps) multiply();
-
-        // the sums of set g >= 1, [block][v][thread of the set], over the staged tiles of A
-        constexpr int SetSums = WBM * WBN * 16 * Threads;
-        static_assert((KGroups - 1) * SetSums * 4 <= KGroups * 3 * PlaneA * 2, "the sets' sums fit the staged tiles");
-        float* const sums = reinterpret_cast<float*>(staged_a) + t;
-        __syncthreads();
-        if (group > 0) {
-            float* out = sums + (group - 1) * SetSums;
-#pragma unroll
-            for (int i = 0; i < WBM; ++i)
-#pragma unroll
-                for (int j = 0; j < WBN; ++j)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) out[((i * WBN + j) * 16 + v) * Threads] = acc[i][j][v];
-        }
-        __syncthreads();
-        if (group > 0) return;
-#pragma unroll
-        for (int g = 1; g < KGroups; ++g) {
-            const float* in = sums + (g - 1) * SetSums;
-#pragma unroll
-            for (int i = 0; i < WBM; ++i)
-#pragma unroll
-                for (int j = 0; j < WBN; ++j)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) acc[i][j][v] += in[((i * WBN + j) * 16 + v) * Threads];
-        }
+        stage();
     }
+    if (full > 0 && tail > 0) {
+        la.load_tail(A, p.lda, tail);
+        lb.load_tail(B, p.ldb, tail);
+        __syncthreads();
+        multiply();
+        __syncthreads();
+        stage();
+    }
+    __syncthreads();
+    multiply();
 
     if (row_sums) {
         // thread t holds the partial sums of row t % TM over its groups: add the groups in K order
@@ -430,42 +365,22 @@ __global__ __launch_bounds__(WGM * WGN * kWave * KGroups) __attribute__((amdgpu_
 // which waste less of a tile (24576 x 37 x 128, batch 2: 15.1 us against 10.1 us).
 constexpr long long kWideTiles = 256;
 
-// Sets of waves per 64 x 64 tile.  With at most one tile per CU a SIMD holds one wave of a set, and its chain of
-// split, LDS round trip and products repeats for every 32 of K; more sets run their chains side by side.  A second
-// register set of loads in flight, a second LDS buffer and sets of one or two waves all left the chain as long.
-// Measured, one set -> the rule's choice: four sets from 512 of K, 4096 x 256 x 1024 23.6 -> 20.0 us, 256 x 1024 x 1024
-// (batch 2, weight gradient) 27.5 -> 19.9 us, 4096 x 256 x 512 13.3 -> 12.0 us; two from 256, where the sums' exchange
-// makes four dearer, 4096 x 128 x 256 7.7 -> 7.35 us (four: 7.6); at 128 of K two gain nothing (5.9 us).  With two tiles
-// per CU one set is faster: 1024 x 1024 x 256 (batch 2) 11.7 us, two sets 12.0 us, four 15.5 us.  Products with row
-// sums take one: the sums follow the order of K.
-int k_groups(const Params& p) {
-    const long long tiles = static_cast<long long>(ceil_div(p.m, 64)) * ceil_div(p.n, 64) * p.batch * p.splits;
-    const int depth = std::min(p.k, p.k_per_split);
-    if (p.a_sums || tiles > 256 || depth < 256) return 1;
-    return depth >= 512 ? 4 : 2;
-}
-
 bool split_eligible(const Params& p, bool ak, bool bk) {
     // 32-bit offsets inside a tile, and row sums of an M-contiguous A only
     return p.lda < (1 << 22) && p.ldb < (1 << 22) && p.ldd < (1 << 24) && !(p.a_sums && ak);
 }
 
-template <int T, int WGM, int WGN, int MinWaves, int KGroups, bool AK, bool BK>
+template <int T, int WGM, int WGN, int MinWaves, bool AK, bool BK>
 void launch_split_tiled(const Params& p, hipStream_t stream) {
     const dim3 grid(ceil_div(p.n, T), ceil_div(p.m, T), static_cast<unsigned>(p.batch * p.splits));
-    hipLaunchKernelGGL((split_kernel<T, T, WGM, WGN, 32, MinWaves, KGroups, AK, BK>), grid,
-                       dim3(WGM * WGN * kWave * KGroups), 0, stream, p);
+    hipLaunchKernelGGL((split_kernel<T, T, WGM, WGN, 32, MinWaves, AK, BK>), grid, dim3(WGM * WGN * kWave), 0, stream, p);
 }
 
 template <bool AK, bool BK>
 void launch_split_layout(const Params& p, hipStream_t stream) {
     const long long wide = static_cast<long long>(ceil_div(p.m, 128)) * ceil_div(p.n, 128) * p.batch * p.splits;
-    if (p.m > 64 && p.n > 64 && wide >= kWideTiles) return launch_split_tiled<128, 2, 4, 2, 1, AK, BK>(p, stream);
-    switch (k_groups(p)) {
-    case 4: return launch_split_tiled<64, 2, 2, 4, 4, AK, BK>(p, stream);
-    case 2: return launch_split_tiled<64, 2, 2, 4, 2, AK, BK>(p, stream);
-    default: return launch_split_tiled<64, 2, 2, 4, 1, AK, BK>(p, stream);
-    }
+    if (p.m > 64 && p.n > 64 && wide >= kWideTiles) launch_split_tiled<128, 2, 4, 2, AK, BK>(p, stream);
+    else launch_split_tiled<64, 2, 2, 4, AK, BK>(p, stream);
 }
 
 void launch_split(const Params& p, bool ak, bool bk, hipStream_t stream) {
