@@ -622,8 +622,11 @@ class FlashSAC:
         n = obs.shape[0]
         if training and n != self.num_envs:
             raise ValueError("Training action batches must match num_envs.")
-        A, p = self.action_dim, self.actor_p
+        A, d, p = self.action_dim, self.observation_dim, self.actor_p
+        fused = K.actor_act_fits(n, d, self.cfg.actor_hidden_dim, self.cfg.actor_num_blocks, A)
         with torch.cuda.device(self.device):
+            if not fused or not K.actor_rows_readable(obs, d):
+                obs = obs[:, :d].contiguous()
             noise = None
             if training:
                 _native.call("rl_exploration_noise", self.cfg.seed * 7919 + 37, self.exploration_step.data_ptr(),
@@ -631,14 +634,11 @@ class FlashSAC:
                              self.exploration_state.data_ptr(), self.exploration_noise.data_ptr(), n * A, None, None,
                              K.stream())
                 noise = self.exploration_noise
-            if K.actor_act_fits(n, self.observation_dim, self.cfg.actor_hidden_dim, self.cfg.actor_num_blocks, A):
-                if obs.stride(1) != 1 or obs.stride(0) < self.observation_dim:
-                    obs = obs[:, : self.observation_dim].contiguous()
+            if fused:
                 actions = torch.empty(n, A, device=self.device)
-                K.actor_act(obs, self._act_parameters, noise, actions, obs_dim=self.observation_dim,
-                            hidden=self.cfg.actor_hidden_dim, blocks=self.cfg.actor_num_blocks, action_dim=A)
+                K.actor_act(obs, self._act_parameters, noise, actions, obs_dim=d, hidden=self.cfg.actor_hidden_dim,
+                            blocks=self.cfg.actor_num_blocks, action_dim=A)
                 return actions
-            obs = obs[:, : self.observation_dim].contiguous()
             net, head, actions = self._act_net(n)
             net.forward(p, p, self.actor_running, obs, rows=n, x_stride=0, training=False)
             net.post_norm(p, rows=n, row0=0, count=n)

@@ -363,10 +363,18 @@ def actor_act_fits(rows, obs_dim, hidden, blocks, action_dim) -> bool:
             and weights <= 700_000)
 
 
+def actor_rows_readable(obs, obs_dim) -> bool:
+    """Whether actor_act reads the first obs_dim columns of obs [rows, >= obs_dim] where they are: consecutive values
+    in rows that do not overlap.  The strides of dimensions of size one say nothing (torch calls a [rows, 1] view with
+    strides (1, rows) contiguous, so .contiguous() returns it as it is)."""
+    return (obs_dim == 1 or obs.stride(1) == 1) and (obs.shape[0] <= 1 or obs.stride(0) >= obs_dim)
+
+
 def actor_act(obs, parameters, noise, actions, *, obs_dim, hidden, blocks, action_dim, bn_eps=1e-5, rms_eps=1e-6):
     """The eval-mode actor's actions in one launch (rl_actor_act); obs may have a row pitch."""
     rows = obs.shape[0]
-    if obs.dtype != torch.float32 or not obs.is_cuda or obs.shape[1] < obs_dim or obs.stride(1) != 1:
+    if (obs.dtype != torch.float32 or not obs.is_cuda or obs.dim() != 2 or obs.shape[1] < obs_dim
+            or not actor_rows_readable(obs, obs_dim)):
         raise ValueError("Acting takes float32 GPU observations with contiguous rows.")
     _check(actions, rows * action_dim, "actions")
     _check_optional(noise, rows * action_dim, "exploration noise")

@@ -56,3 +56,44 @@ def test_one_launch_actor_matches_float64(gpu, obs_dim, action_dim, hidden, bloc
     finally:
         K.actor_act_fits = fits
     torch.testing.assert_close(agent.act(observations, training=False), layered, rtol=0, atol=4e-6)
+
+
+# [rows, columns] observations of every stride that .contiguous() may hand on as it is or has to copy
+VIEWS = {
+    "packed": lambda x: x,
+    "transposed": lambda x: x.t().contiguous().t(),
+    "every other row": lambda x: x.repeat_interleave(2, 0)[::2],
+    "every other column": lambda x: x.repeat_interleave(2, 1)[:, ::2],
+    "one row for all": lambda x: x[:1].expand(x.shape[0], -1),
+    "one value for all": lambda x: x[:1, :1].expand(x.shape),
+}
+
+
+@pytest.mark.parametrize("view", VIEWS)
+@pytest.mark.parametrize("rows,obs_dim,columns", [(1, 1, 1), (1, 1, 3), (1, 5, 5), (7, 1, 1), (7, 1, 4), (7, 5, 5), (7, 5, 8)])
+def test_observation_strides(gpu, rows, obs_dim, columns, view):
+    """act() on views of any strides gives what it gives on packed rows, with the same exploration draws."""
+    print(f"case actor strides rows={rows} obs={obs_dim} columns={columns} view={view}", flush=True)
+    cfg = FlashSACConfig(seed=5, actor_hidden_dim=32, actor_num_blocks=1, critic_hidden_dim=32, critic_num_blocks=1,
+                         sample_batch_size=16, buffer_max_length=64, buffer_min_length=16)
+    agent, packed = (FlashSAC(obs_dim, 2, num_envs=rows, cfg=cfg) for _ in range(2))
+    x = VIEWS[view](torch.randn(rows, columns, generator=torch.Generator(device=gpu).manual_seed(rows), device=gpu))
+    same = torch.empty(rows, columns, device=gpu).copy_(x)
+    for training in (False, True, True):
+        assert torch.equal(agent.act(x, training=training), packed.act(same, training=training))
+    assert int(agent.exploration_step) == int(packed.exploration_step)
+
+
+def test_refused_observations_draw_no_noise(gpu):
+    cfg = FlashSACConfig(seed=5, actor_hidden_dim=32, actor_num_blocks=1, critic_hidden_dim=32, critic_num_blocks=1,
+                         sample_batch_size=16, buffer_max_length=64, buffer_min_length=16)
+    agent = FlashSAC(3, 2, num_envs=4, cfg=cfg)
+    for shape in ((4,), (4, 2), (3, 3), (4, 3, 1)):
+        with pytest.raises(ValueError):
+            agent.act(torch.zeros(shape, device=gpu), training=True)
+    assert int(agent.exploration_step) == 0
+    # overlapping rows are refused where a copy is not made for the caller
+    rows = torch.zeros(1, 3, device=gpu).expand(4, 3)
+    with pytest.raises(ValueError):
+        K.actor_act(rows, agent._act_parameters, None, torch.empty(4, 2, device=gpu), obs_dim=3, hidden=32, blocks=1,
+                    action_dim=2)
