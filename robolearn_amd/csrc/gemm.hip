@@ -679,7 +679,7 @@ int run_gemm(int mode, int a_bf16, int b_bf16, int a_kcontig, int b_kcontig, int
     p.moments = fused_moments ? moments : nullptr;
     if (mode == 1) gemm::launch_bf16(p, a_bf16, b_bf16, a_kcontig != 0, b_kcontig != 0, stream);
     else if (mode == 3) gemm::launch_f16(p, a_bf16, b_bf16, a_kcontig != 0, b_kcontig != 0, stream);
-    else if (mode == 2 && gemm::split_eligible(p, a_kcontig != 0, b_kcontig != 0))
+    else if (mode == 2 && gemm::split_eligible(p, a_kcontig != 0))
         gemm::launch_split(p, a_kcontig != 0, b_kcontig != 0, stream);
     else gemm::launch_fp32(p, a_kcontig != 0, b_kcontig != 0, stream);
     check_launch("Launch GEMM");

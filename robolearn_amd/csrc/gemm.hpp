@@ -57,8 +57,8 @@ __device__ __forceinline__ float apply_epilogue(float v, int epilogue) {
     return v;
 }
 
-// fp32 products from three bf16 pieces per operand value (gemm_split.hip); split_eligible: the layouts it takes.
-bool split_eligible(const Params& p, bool ak, bool bk);
+// fp32 products from three bf16 pieces per operand value (gemm_split.hip); split_eligible: the products it takes.
+bool split_eligible(const Params& p, bool ak);
 void launch_split(const Params& p, bool ak, bool bk, hipStream_t stream);
 
 // bf16 MFMA kernel family with 256x128 tiles (gemm_bf16.hip).

@@ -53,14 +53,14 @@ __device__ __forceinline__ int slot(int r, int c) {
 // One Rows x Step operand tile, held in registers between its load and its store to LDS.  Element (r, k) of
 // the operand is src[r * ld + k] when KContig, else src[k * ld + r].  Rows past the operand's end repeat its
 // last row: their products land in output rows that are not written.
-template <bool KContig, int Rows, int Threads, int Step>
+template <bool KContig, int Rows, int Threads, int Step, class Offset>
 struct SplitLoader {
     static constexpr int Vec = Step / 4;                  // K-contiguous: float4 per row
     static constexpr int Count = Rows * Step / Threads;   // values per thread
     static constexpr int Owned = KContig ? Count / 4 : 1; // rows this thread holds values of
     float regs[Count];
-    unsigned offset[Owned];  // byte offset of this thread's values in the tile
-    int k_first;             // M/N-contiguous: first K of this thread
+    Offset offset[Owned];  // byte offset of this thread's values in the tile
+    int k_first;           // M/N-contiguous: first K of this thread
 
     __device__ __forceinline__ int row(int i) const {
         const int t = static_cast<int>(threadIdx.x);
@@ -71,14 +71,14 @@ struct SplitLoader {
         const int t = static_cast<int>(threadIdx.x);
 #pragma unroll
         for (int i = 0; i < Owned; ++i) {
-            const unsigned r = static_cast<unsigned>(min(row(i), rows - 1));
-            offset[i] = KContig ? (r * static_cast<unsigned>(ld) + (t % Vec) * 4u) * 4u : r * 4u;
+            const Offset r = static_cast<Offset>(min(row(i), rows - 1));
+            offset[i] = KContig ? (r * static_cast<Offset>(ld) + (t % Vec) * 4u) * 4u : r * 4u;
         }
         // uniform over a wave (Rows is a multiple of 64)
         k_first = KContig ? 0 : __builtin_amdgcn_readfirstlane(t / Rows) * Count;
     }
 
-    __device__ __forceinline__ static const float* at(const float* p, unsigned bytes) {
+    __device__ __forceinline__ static const float* at(const float* p, Offset bytes) {
         return reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + bytes);
     }
 
@@ -148,7 +148,8 @@ struct SplitLoader {
 
 // TM x TN output tile of WGM x WGN waves; MinWaves: the waves per SIMD the register allocation aims at (the 128
 // x 128 kernels fit 128 registers, so four waves, under a bound of 2 too, with better schedules: 99.4 -> 96.3 us).
-template <int TM, int TN, int WGM, int WGN, int Step, int MinWaves, bool AK, bool BK>
+// Offset: of a value in its tile, unsigned where that holds a tile's rows at their pitch.
+template <int TM, int TN, int WGM, int WGN, int Step, int MinWaves, class Offset, bool AK, bool BK>
 __global__ __launch_bounds__(WGM * WGN * kWave) __attribute__((amdgpu_waves_per_eu(MinWaves))) void split_kernel(
     Params p) {
     constexpr int Threads = WGM * WGN * kWave;
@@ -189,8 +190,8 @@ __global__ __launch_bounds__(WGM * WGN * kWave) __attribute__((amdgpu_waves_per_
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
 
-    SplitLoader<AK, TM, Threads, Step> la;
-    SplitLoader<BK, TN, Threads, Step> lb;
+    SplitLoader<AK, TM, Threads, Step, Offset> la;
+    SplitLoader<BK, TN, Threads, Step, Offset> lb;
     la.init(p.lda, p.m - m0);
     lb.init(p.ldb, p.n - n0);
 
@@ -320,7 +321,7 @@ __global__ __launch_bounds__(WGM * WGN * kWave) __attribute__((amdgpu_waves_per_
 #pragma unroll
         for (int j = 0; j < WBN; ++j) {
             const int col = wn * WTN + j * 32 + lane % 32;
-            const unsigned offset = static_cast<unsigned>(wave_row) * static_cast<unsigned>(ldd) + col;
+            const Offset offset = static_cast<Offset>(wave_row) * static_cast<Offset>(ldd) + col;
             const bool in_n = whole || n0 + col < p.n;
             const auto in = [&](int v) { return whole || (in_n && m0 + wave_row + i * 32 + 8 * (v / 4) + v % 4 < p.m); };
             // all C values are loaded before the first store: the compiler cannot tell C from D apart, and a
@@ -365,22 +366,30 @@ __global__ __launch_bounds__(WGM * WGN * kWave) __attribute__((amdgpu_waves_per_
 // which waste less of a tile (24576 x 37 x 128, batch 2: 15.1 us against 10.1 us).
 constexpr long long kWideTiles = 256;
 
-bool split_eligible(const Params& p, bool ak, bool bk) {
-    // 32-bit offsets inside a tile, and row sums of an M-contiguous A only
-    return p.lda < (1 << 22) && p.ldb < (1 << 22) && p.ldd < (1 << 24) && !(p.a_sums && ak);
-}
+// Row sums are those of an M-contiguous A only.
+bool split_eligible(const Params& p, bool ak) { return !(p.a_sums && ak); }
 
-template <int T, int WGM, int WGN, int MinWaves, bool AK, bool BK>
+template <int T, int WGM, int WGN, int MinWaves, class Offset, bool AK, bool BK>
 void launch_split_tiled(const Params& p, hipStream_t stream) {
     const dim3 grid(ceil_div(p.n, T), ceil_div(p.m, T), static_cast<unsigned>(p.batch * p.splits));
-    hipLaunchKernelGGL((split_kernel<T, T, WGM, WGN, 32, MinWaves, AK, BK>), grid, dim3(WGM * WGN * kWave), 0, stream, p);
+    hipLaunchKernelGGL((split_kernel<T, T, WGM, WGN, 32, MinWaves, Offset, AK, BK>), grid, dim3(WGM * WGN * kWave), 0,
+                       stream, p);
 }
 
+template <class Offset, bool AK, bool BK>
+void launch_split_offset(const Params& p, hipStream_t stream) {
+    const long long wide = static_cast<long long>(ceil_div(p.m, 128)) * ceil_div(p.n, 128) * p.batch * p.splits;
+    if (p.m > 64 && p.n > 64 && wide >= kWideTiles) launch_split_tiled<128, 2, 4, 2, Offset, AK, BK>(p, stream);
+    else launch_split_tiled<64, 2, 2, 4, Offset, AK, BK>(p, stream);
+}
+
+// 32-bit offsets hold 128 rows of fewer than 2^22 values in bytes (an M/N-contiguous operand's rows are adjacent
+// whatever its pitch) and 128 output rows of fewer than 2^24 in values; partial sums are p.n apart.
 template <bool AK, bool BK>
 void launch_split_layout(const Params& p, hipStream_t stream) {
-    const long long wide = static_cast<long long>(ceil_div(p.m, 128)) * ceil_div(p.n, 128) * p.batch * p.splits;
-    if (p.m > 64 && p.n > 64 && wide >= kWideTiles) launch_split_tiled<128, 2, 4, 2, AK, BK>(p, stream);
-    else launch_split_tiled<64, 2, 2, 4, AK, BK>(p, stream);
+    const bool near = (!AK || p.lda < (1 << 22)) && (!BK || p.ldb < (1 << 22)) && (p.splits > 1 || p.ldd < (1 << 24));
+    if (near) launch_split_offset<unsigned, AK, BK>(p, stream);
+    else launch_split_offset<unsigned long long, AK, BK>(p, stream);
 }
 
 void launch_split(const Params& p, bool ak, bool bk, hipStream_t stream) {

@@ -705,3 +705,42 @@ def test_fp32_split_products_over_the_exponent_range(gpu, m, n, k, splits, a_kco
         total = a64.sum(1)
         slack = a64.abs().sum(1) * (8 + splits) * 2.0**-23
         assert ((sums.cpu().double()[rows] - total).abs() <= slack).all()
+
+
+# operands and outputs whose rows lie too far apart for 32-bit offsets inside a tile: pitches at and beside the limits
+# (2^22 values of an operand, 2^24 of D), members and splits on 64- and on 128-wide tiles
+@pytest.mark.parametrize("a_kcontig,b_kcontig", [(True, True), (True, False), (False, True), (False, False)])
+@pytest.mark.parametrize("far", ["a", "b", "d"])
+@pytest.mark.parametrize("beyond", [-1, 0, 1])
+@pytest.mark.parametrize("m,n,k,batch,splits", [(65, 33, 40, 1, 1), (33, 130, 70, 2, 3), (66, 65, 24, 256, 1)])
+def test_fp32_split_products_of_far_rows(gpu, m, n, k, batch, splits, beyond, far, a_kcontig, b_kcontig):
+    """Mode 2 gives the bits that it gives on packed rows, row sums and C included."""
+    print(f"case split far={far}{beyond:+d} m={m} n={n} k={k} batch={batch} splits={splits} ak={a_kcontig} bk={b_kcontig}",
+          flush=True)
+    g = torch.Generator(device=gpu).manual_seed(m + n)
+
+    def laid_out(rows, cols, pitch, values=None):
+        """[batch, rows, cols] with the members side by side in rows `pitch` apart (packed: pitch None)."""
+        if pitch is None:
+            out = torch.empty(batch, rows, cols, device=gpu)
+        else:
+            out = torch.empty((rows - 1) * pitch + batch * cols, device=gpu).as_strided((batch, rows, cols), (cols, pitch, 1))
+        return out if values is None else out.copy_(values)
+
+    shapes = {"a": (m, k) if a_kcontig else (k, m), "b": (n, k) if b_kcontig else (k, n), "d": (m, n)}
+    values = {key: torch.randn(batch, *shape, generator=g, device=gpu) for key, shape in shapes.items()}
+    workspace = torch.empty(splits * batch * (m * n + m) * 4, dtype=torch.uint8, device=gpu) if splits > 1 else None
+    results = []
+    for pitch in (None, (1 << (24 if far == "d" else 22)) + beyond):
+        t = {key: laid_out(*shapes[key], pitch if key == far else None, values[key]) for key in "ab"}
+        c = laid_out(m, n, pitch if far == "d" else None, values["d"])
+        sums = None if a_kcontig else torch.empty(batch, m, device=gpu)
+        # in place: D is C
+        K.gemm(t["a"], t["b"], c, m=m, n=n, k=k, batch=batch, a_kcontig=a_kcontig, b_kcontig=b_kcontig,
+               lda=t["a"].stride(1), ldb=t["b"].stride(1), ldd=c.stride(1), stride_a=t["a"].stride(0),
+               stride_b=t["b"].stride(0), stride_d=c.stride(0), c=c, beta=0.5, mode=K.FP32_SPLIT, splits=splits,
+               workspace=workspace, a_sums=sums)
+        results.append((c.clone(memory_format=torch.contiguous_format), sums))
+    assert torch.equal(results[0][0], results[1][0])
+    if not a_kcontig:
+        assert torch.equal(results[0][1], results[1][1])
