@@ -463,6 +463,13 @@ int fp32_tile(const Params& p) {
     return big >= 2048 ? 128 : 64;
 }
 
+const char* kernel_name(int mode, const Params& p, int a_16bit, int b_16bit) {
+    if (mode == 0) return fp32_tile(p) == 128 ? "mfma_128x128" : "mfma_64x64";
+    if (mode == 1 && big_eligible(p, a_16bit, b_16bit)) return "mfma_256x256";
+    if (mode == 1 && narrow_eligible(p, a_16bit, b_16bit)) return "mfma_64x64";
+    return "mfma_256x128";
+}
+
 template <int T, bool AK, bool BK>
 void launch_fp32_tiled(const Params& p, hipStream_t stream) {
     const dim3 grid(ceil_div(p.n, T), ceil_div(p.m, T), static_cast<unsigned>(p.batch * p.splits));
@@ -642,13 +649,8 @@ int run_gemm(int mode, int a_bf16, int b_bf16, int a_kcontig, int b_kcontig, int
     p.beta = beta;
     p.epilogue = epilogue;
     p.d_bf16 = d_bf16;
-    const int kt = half_mode ? 32 : 16;
-    const int ktiles = (k + kt - 1) / kt;
-    if (splits > ktiles) splits = ktiles;
-    const int tiles_per_split = (ktiles + splits - 1) / splits;  // split boundaries are multiples of 32 in both modes
-    splits = (ktiles + tiles_per_split - 1) / tiles_per_split;
+    p.k_per_split = gemm::split_depth(mode, k, splits);
     p.splits = splits;
-    p.k_per_split = tiles_per_split * kt;
     const std::size_t a_elem = a_bf16 ? 2 : 4;
     const std::size_t b_elem = b_bf16 ? 2 : 4;
     p.a_vec = aligned(a, 16) && (lda * a_elem) % 16 == 0 && (stride_a * a_elem) % 16 == 0;
@@ -743,11 +745,7 @@ RL_API int rl_gemm(int mode, int a_bf16, int b_bf16, int a_kcontig, int b_kconti
 
 RL_API std::size_t rl_gemm_workspace(int mode, int m, int n, int k, int batch, int splits) noexcept {
     if (m <= 0 || n <= 0 || k <= 0 || batch <= 0 || splits <= 1) return 0;
-    const int kt = (mode == 1 || mode == 3) ? 32 : 16;
-    const int ktiles = (k + kt - 1) / kt;
-    if (splits > ktiles) splits = ktiles;
-    const int per = (ktiles + splits - 1) / splits;
-    splits = (ktiles + per - 1) / per;
+    rl::gemm::split_depth(mode, k, splits);
     if (splits <= 1) return 0;
     // D partials plus the row-sum partials of A
     return static_cast<std::size_t>(splits) * batch * (static_cast<std::size_t>(m) * n + m) * sizeof(float);

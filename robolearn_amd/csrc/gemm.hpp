@@ -57,6 +57,19 @@ __device__ __forceinline__ float apply_epilogue(float v, int epilogue) {
     return v;
 }
 
+// K of one split, a multiple of the mode's K tile; lowers splits to those that have any K.
+inline int split_depth(int mode, int k, int& splits) {
+    const int kt = mode == 1 || mode == 3 ? 32 : 16;
+    const int ktiles = (k + kt - 1) / kt;
+    if (splits > ktiles) splits = ktiles;
+    const int per = (ktiles + splits - 1) / splits;
+    splits = (ktiles + per - 1) / per;
+    return per * kt;
+}
+
+// The output tile of the kernel that runs p in this mode (a_16bit, b_16bit: 16-bit operand storage).
+const char* kernel_name(int mode, const Params& p, int a_16bit, int b_16bit);
+
 // fp32 products from three bf16 pieces per operand value (gemm_split.hip); split_eligible: the products it takes.
 bool split_eligible(const Params& p, bool ak);
 void launch_split(const Params& p, bool ak, bool bk, hipStream_t stream);

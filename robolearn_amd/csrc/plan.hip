@@ -70,8 +70,23 @@ void* create_plan(int m, int n, int k, int transa, int transb, int lda, int ldb,
     }
     plan->splits = splits;
     plan->workspace_bytes = bytes;
+    // the row-major view that rl_plan_run multiplies, on buffers aligned to 16 bytes
+    rl::gemm::Params p{};
+    p.m = n;
+    p.n = m;
+    p.k = k;
+    p.batch = 1;
+    p.lda = ldb;
+    p.ldb = lda;
+    p.ldd = ldd;
+    p.splits = splits;
+    p.k_per_split = rl::gemm::split_depth(plan->mode, k, p.splits);
+    const int operand_bytes = plan->operands_16bit ? 2 : 4;
+    p.a_vec = p.lda * operand_bytes % 16 == 0;
+    p.b_vec = p.ldb * operand_bytes % 16 == 0;
+    const char* kernel = rl::gemm::kernel_name(plan->mode, p, plan->operands_16bit, plan->operands_16bit);
     const char* precision = plan->mode == 0 ? "fp32" : (plan->mode == 3 ? "fp16" : "bf16");
-    plan->metadata = "{\"kernel\":\"" + std::string(plan->mode ? "mfma_256x128" : "mfma_128x128") +
+    plan->metadata = "{\"kernel\":\"" + std::string(kernel) +
                      "\",\"mode\":\"" + std::string(precision) +
                      "\",\"split_k\":" + std::to_string(splits) + ",\"workspace_bytes\":" + std::to_string(bytes) +
                      ",\"autotuned\":false}";

@@ -64,3 +64,31 @@ def test_dense_plan_metadata_and_workspace_on_host():
 def test_exports_have_c_linkage():
     library = ctypes.CDLL(str(_native.library_path()))
     assert library.rl_last_error is not None
+
+
+def plan_kernel(rows, cols, k, input_dtype, transa=1, transb=0, workspace=64 << 20):
+    """The metadata's kernel for a row-major [rows, cols] product over k (the plan's view is its transpose)."""
+    import json
+
+    library = _native.load()
+    plan = _native.create("rl_plan_create_mixed", cols, rows, k, transa, transb, k if transa else cols,
+                          k if transb == 0 else rows, cols, 0, 0, input_dtype, workspace)
+    metadata = json.loads(library.rl_plan_tuning_metadata(plan).decode())
+    assert library.rl_plan_destroy(plan) == 0
+    return metadata["kernel"]
+
+
+@pytest.mark.parametrize("rows,cols,k,input_dtype,kernel", [
+    (2048, 101, 512, 3, "mfma_64x64"),        # a head
+    (4096, 512, 39, 3, "mfma_64x64"),         # an embedder
+    (1, 1, 1, 3, "mfma_64x64"),
+    (16384, 4096, 1024, 3, "mfma_256x256"),   # a block layer
+    (16384, 4000, 1000, 3, "mfma_256x128"),   # the same, ragged
+    (16384, 4000, 1000, 2, "mfma_256x128"),   # fp32 operands rounded on load
+    (2048, 101, 512, 2, "mfma_256x128"),
+    (2048, 101, 512, 1, "mfma_256x128"),      # fp16
+    (64, 64, 64, 0, "mfma_64x64"),
+    (16384, 4096, 1024, 0, "mfma_128x128"),
+])
+def test_dense_plan_metadata_names_the_kernel(rows, cols, k, input_dtype, kernel):
+    assert plan_kernel(rows, cols, k, input_dtype) == kernel
