@@ -463,10 +463,10 @@ int fp32_tile(const Params& p) {
     return big >= 2048 ? 128 : 64;
 }
 
-const char* kernel_name(int mode, const Params& p, int a_16bit, int b_16bit) {
+const char* kernel_name(int mode, const Params& p, int a_16bit, int b_16bit, bool ak, bool bk) {
     if (mode == 0) return fp32_tile(p) == 128 ? "mfma_128x128" : "mfma_64x64";
     if (mode == 1 && big_eligible(p, a_16bit, b_16bit)) return "mfma_256x256";
-    if (mode == 1 && narrow_eligible(p, a_16bit, b_16bit)) return "mfma_64x64";
+    if (mode == 1 && narrow_eligible(p, a_16bit, b_16bit, ak, bk)) return "mfma_64x64";
     return "mfma_256x128";
 }
 

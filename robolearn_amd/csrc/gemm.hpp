@@ -68,7 +68,7 @@ inline int split_depth(int mode, int k, int& splits) {
 }
 
 // The output tile of the kernel that runs p in this mode (a_16bit, b_16bit: 16-bit operand storage).
-const char* kernel_name(int mode, const Params& p, int a_16bit, int b_16bit);
+const char* kernel_name(int mode, const Params& p, int a_16bit, int b_16bit, bool ak, bool bk);
 
 // fp32 products from three bf16 pieces per operand value (gemm_split.hip); split_eligible: the products it takes.
 bool split_eligible(const Params& p, bool ak);
@@ -80,8 +80,8 @@ void launch_bf16(const Params& p, int a_bf16, int b_bf16, bool ak, bool bk, hipS
 // else fp32 rounded to fp16 on load).
 void launch_f16(const Params& p, int a_f16, int b_f16, bool ak, bool bk, hipStream_t stream);
 
-// 64x64-tile bf16 kernel for narrow or small products (gemm_bf16_narrow.hip).
-bool narrow_eligible(const Params& p, int a_bf16, int b_bf16);
+// 64x64-tile bf16 kernel for narrow, small or unaligned products (gemm_bf16_narrow.hip).
+bool narrow_eligible(const Params& p, int a_bf16, int b_bf16, bool ak, bool bk);
 void launch_narrow(const Params& p, bool ak, bool bk, hipStream_t stream);
 
 // 256x256-tile bf16 kernel for exactly tiling bf16 operands (gemm_bf16_big.hip).

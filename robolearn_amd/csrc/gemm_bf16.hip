@@ -376,7 +376,7 @@ void launch_bf16(const Params& p, int a_bf16, int b_bf16, bool ak, bool bk, hipS
         launch_big(p, ak, bk, stream);
         return;
     }
-    if (narrow_eligible(p, a_bf16, b_bf16)) {
+    if (narrow_eligible(p, a_bf16, b_bf16, ak, bk)) {
         launch_narrow(p, ak, bk, stream);
         return;
     }

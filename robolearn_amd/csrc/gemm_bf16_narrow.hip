@@ -260,19 +260,34 @@ void launch(const Params& p, hipStream_t stream) {
 
 }  // namespace narrow
 
-// Where 256 x 128 tiles give every CU more than one workgroup and K is deep, their four times larger operand reuse
-// wins (twin, 6000 x 4000 over 1000: 190 us against 307 us; 6000 x 1000 over 4000, 384 tiles: 159 us against 203
-// us); with fewer tiles or a shorter K the small ones do (8192 x 640 over 2560, 320 tiles: 108 us against 97 us;
-// 8192 x 2560 over 640, 1280 tiles: 137 us against 136 us).
-constexpr long long kWideTiles = 384;
-constexpr int kWideDepth = 768;
+// One round of 256 x 128 tiles (512: two workgroups per CU, however few of them the last round fills) takes about as
+// long as 1500 of the small ones, whose operand reuse is four times smaller, or as 1800 where an operand is M- or
+// N-contiguous and the large tiles transpose it; the additions to K are what a tile costs before and after its K loop.
+// The line is fitted to 1516 random products of 128 large tiles and more (24 to 20000 rows and columns, K from 24 to
+// 16000, all layouts, whole and split).  Of the 679 that it gives the small tiles 35 are 3 to 15 % slower there and the
+// others up to 3.9 times faster; of the 837 that it leaves to the large tiles 429 would take up to 2.2 times as long on
+// small ones and 244 would be 5 to 60 % faster.  With fewer large tiles the small ones always won (1.18 to 5.8 times
+// faster).  500 x 16000 over 1000, twin: 100 us on small tiles, 64 on
+// large ones; 16400 x 400 over 8200 421 and 335 us; 16384 x 1024 over 160, twin 43 and 46 us; 4096 x 512 over 160, twin
+// 10.1 and 17.6 us.
+// Operands that do not load 16 bytes at a time, which the large tiles read one value at a time, take the small tiles at
+// any size: 1.07 to 26 times faster, 3.2 times in the middle, in 1443 random products (3190 x 4972 over 29 is 13 %
+// slower); 2396 x 567 over 12951 in four splits, twin: 214 against 919 us.
+constexpr int kRowTilesPerRound = 1500, kTransposedTilesPerRound = 1800;
+constexpr int kWideRound = 512;
+constexpr int kNarrowFixed = 128, kWideFixed = 256;
 
-bool narrow_eligible(const Params& p, int a_bf16, int b_bf16) {
-    const long long wide = static_cast<long long>(ceil_div(p.m, 256)) * ceil_div(p.n, 128) * p.batch * p.splits;
-    if (p.m > 512 && p.n > 512 && wide >= kWideTiles && p.k_per_split >= kWideDepth) return false;
+bool narrow_eligible(const Params& p, int a_bf16, int b_bf16, bool ak, bool bk) {
+    const long long products = static_cast<long long>(p.batch) * p.splits;
     const long long rows = ceil_div(p.m, narrow::kTileEdge);
-    // 32-bit offsets inside a tile
-    return a_bf16 && b_bf16 && p.lda < (1 << 22) && p.ldb < (1 << 22) && rows <= 65535 && p.batch * p.splits <= 65535;
+    // 32-bit offsets inside a tile, and the grid's limits
+    if (!a_bf16 || !b_bf16 || p.lda >= (1 << 22) || p.ldb >= (1 << 22) || rows > 65535 || products > 65535) return false;
+    if (!p.a_vec || !p.b_vec) return true;
+    const long long tiles = rows * ceil_div(p.n, narrow::kTileEdge) * products;
+    const long long wide = static_cast<long long>(ceil_div(p.m, 256)) * ceil_div(p.n, 128) * products;
+    const long long rounds = (wide + kWideRound - 1) / kWideRound;
+    const long long per_round = ak && bk ? kRowTilesPerRound : kTransposedTilesPerRound;
+    return tiles * (p.k_per_split + kNarrowFixed) < per_round * rounds * (p.k_per_split + kWideFixed);
 }
 
 void launch_narrow(const Params& p, bool ak, bool bk, hipStream_t stream) {

@@ -92,3 +92,22 @@ def plan_kernel(rows, cols, k, input_dtype, transa=1, transb=0, workspace=64 << 
 ])
 def test_dense_plan_metadata_names_the_kernel(rows, cols, k, input_dtype, kernel):
     assert plan_kernel(rows, cols, k, input_dtype) == kernel
+
+
+# either side of the line in rows, K, rounds of large tiles and 16-byte rows of the operands; (500, 16000, 1000) takes 64 us
+# on the 256 x 128 tiles and 100 us on the 64 x 64 ones as a twin product
+@pytest.mark.parametrize("rows,cols,k,transa,transb,kernel", [
+    (500, 16000, 1000, 1, 0, "mfma_256x128"),
+    (300, 16000, 1000, 1, 0, "mfma_64x64"),
+    (500, 16000, 1001, 1, 0, "mfma_64x64"),
+    (500, 16000, 16000, 1, 0, "mfma_256x128"),
+    (16400, 400, 8200, 1, 0, "mfma_256x128"),
+    (16400, 504, 8200, 0, 0, "mfma_256x128"),
+    (16401, 400, 8200, 0, 1, "mfma_64x64"),
+    (3000, 3000, 3000, 1, 0, "mfma_256x128"),
+    (3000, 3000, 40, 1, 0, "mfma_64x64"),
+    (16400, 16400, 264, 0, 1, "mfma_256x128"),
+    (24, 16000, 1000, 1, 0, "mfma_64x64"),
+])
+def test_bf16_products_take_the_faster_tiles(rows, cols, k, transa, transb, kernel):
+    assert plan_kernel(rows, cols, k, 3, transa, transb) == kernel
