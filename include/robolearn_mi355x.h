@@ -331,7 +331,7 @@ int rl_exploration_noise(unsigned long long seed, long long* step, const float* 
  * per block W1 [4 hidden, hidden] and its norm (four pointers), W2 [hidden, 4 hidden] and
  * its norm, then the post-norm weight, the mean and log-std head rows [2 action_dim,
  * hidden] and their bias [2 action_dim].  hidden and 2 * action_dim up to 256, obs_dim up
- * to 1024 (512 with hidden <= 128), blocks up to 8.  Replaces the act path of
+ * to 1024, blocks up to 8.  Replaces the act path of
  * robolearn/flashsac/agent.py:414-455 (networks.py:37-61, layers.py:67-166). */
 int rl_actor_act(long long rows, int obs_dim, int hidden, int blocks, int action_dim, const float* obs,
                  long long ld_obs, const void* const* parameters, const float* noise, float* actions, float bn_eps,

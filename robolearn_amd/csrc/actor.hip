@@ -6,12 +6,14 @@
 // output columns, 16 at a time.
 //
 // What bounds it: the weights' way into one CU, about 30 GB/s however many rows (its misses in flight; with the
-// weights in L1 the 256-wide network takes 83 instead of 134 us, at an fp32 matrix floor of 57 us).  So it is the
-// faster way where the layer-by-layer path is all launches: acting alone, observations to actions (layer by layer
-// in brackets), obs 4, hidden 128, one block, 64 rows 22 us (98 us eager, 49 us of it on the GPU); obs 17, hidden 64,
-// 4096 rows 13 us (101, 47); obs 60, hidden 200, two blocks, 4096 rows 87 us (133, 129); obs 123, hidden 256, two
-// blocks 134 us (133 eager, 107 on the GPU, up to 1024 rows), where the caller takes the layers.  Eight waves and
-// deeper prefetch (two to eight chunks, copied or in turn) were no faster.
+// weights in L1 the 256-wide network of two blocks takes 83 instead of 134 us, at an fp32 matrix floor of 57 us).  So
+// it is the faster way where the layer-by-layer path is all launches: observations to actions, one launch against the
+// layers issued one by one / captured in a graph, obs 4, hidden 128, one block, 64 rows 22 us against 98 / 43; obs 17,
+// hidden 64, one block, 4096 rows 13 us against 108 / 42; obs 60, hidden 200, two blocks, 64 rows 85 us against 140 /
+// 90 and 4096 rows 87 us against 137 / 122; obs 123, hidden 256, two blocks, 1024 rows 134 us against 157 / 110, where
+// the caller takes the layers.  Both instances use the 128 registers that sixteen waves leave each other and spill
+// three (16 bytes of scratch a lane).  Eight waves and deeper prefetch (two to eight chunks, copied or in turn) were
+// no faster.
 #include "common.hpp"
 
 #include <cmath>
@@ -26,7 +28,6 @@ constexpr int kRows = 16;
 constexpr int kWaves = 16;
 constexpr int kThreads = kWaves * kWave;
 constexpr int kMaxBlocks = 8;
-
 
 struct Norm {
     const float *mean, *var, *w, *b;

@@ -1,4 +1,6 @@
-// bf16 MFMA GEMM with 256x128 output tiles for the dense-layer products.
+// bf16 MFMA GEMM with 256x128 output tiles for the dense-layer products: ragged bf16 products large enough to fill
+// rounds of such tiles (narrow_eligible in gemm_bf16_narrow.hip draws the line), products with fp32-stored operands, and
+// every fp16 product.
 //
 // Same row-major contract as the fp32 family in gemm.hip (forward, input and
 // weight gradients of a bias-free Linear, batched over ensemble members), tuned

@@ -7,8 +7,8 @@
 // small workgroups overlap each other's chains, and rows load 16 bytes (M/N-contiguous ones, pairs of rows, 4
 // bytes) at any even address.  Twin critics, 256 x 128 tiles against these, bit-identical: 4096 x 512 over K = 39
 // 20.1 -> 9.7 us, 2048 x 101 over 512 with its split 21.3 -> 11.7 us, 101 x 512 over 2048 with its split 21.7 -> 11.6 us,
-// 4096 x 39 over 512 23.5 -> 11.4 us; 16384 x 1024 over 160 53.7 -> 51.6 us, 101 x 1024 over 8192 50.5 -> 27.8 us,
-// 16384 x 160 over 1024 52.8 -> 39.8 us; one member, 16384 x 256 over 123 31.3 -> 10.8 us.
+// 4096 x 39 over 512 23.5 -> 11.4 us; 101 x 1024 over 8192 50.5 -> 27.8 us, 16384 x 160 over 1024 52.8 -> 39.8 us; one
+// member, 16384 x 256 over 123 31.3 -> 10.8 us.
 #include "gemm.hpp"
 
 namespace rl {
@@ -267,9 +267,8 @@ void launch(const Params& p, hipStream_t stream) {
 // 16000, all layouts, whole and split).  Of the 679 that it gives the small tiles 35 are 3 to 15 % slower there and the
 // others up to 3.9 times faster; of the 837 that it leaves to the large tiles 429 would take up to 2.2 times as long on
 // small ones and 244 would be 5 to 60 % faster.  With fewer large tiles the small ones always won (1.18 to 5.8 times
-// faster).  500 x 16000 over 1000, twin: 100 us on small tiles, 64 on
-// large ones; 16400 x 400 over 8200 421 and 335 us; 16384 x 1024 over 160, twin 43 and 46 us; 4096 x 512 over 160, twin
-// 10.1 and 17.6 us.
+// faster).  500 x 16000 over 1000, twin: 100 us on small tiles, 64 on large ones; 16400 x 400 over 8200 421 and 335 us;
+// 16384 x 1024 over 160, twin 43 and 46 us; 4096 x 512 over 160, twin 10.1 and 17.6 us.
 // Operands that do not load 16 bytes at a time, which the large tiles read one value at a time, take the small tiles at
 // any size: 1.07 to 26 times faster, 3.2 times in the middle, in 1443 random products (3190 x 4972 over 29 is 13 %
 // slower); 2396 x 567 over 12951 in four splits, twin: 214 against 919 us.

@@ -6,12 +6,14 @@
 // product is as accurate as an fp32 one, at 6 x 32 matrix-core cycles per 16-K step instead of 8 x 64
 // (v_mfma_f32_32x32x2_f32).
 //
-// What bounds it: the matrix cores reach about 1.0 PFLOP/s of bf16 products here with random operands (1.4
-// with zeros: the difference is power), and between two barriers a wave's split and its products do not
-// overlap, so each is covered only by the other waves of its SIMD (four).  The K loop loads whole steps without
-// bounds checks (rows past the end repeat the last row, the short last step is peeled off), 16 bytes at a
-// time whatever the rows' alignment, and stages unpadded XOR-swizzled rows; the epilogue branches once per
-// block and stores through a uniform base plus a 32-bit lane offset.  Measured against the same tiles with
+// What bounds it: this kernel issues 1.0 to 1.2 PFLOP/s of bf16 products on random operands and 1.3 to 1.5 on zeros
+// or constants (24576 x 512 over 512 and over 2048, batch 2: 150 and 529 us against 108 and 398; the difference is
+// power), and between two barriers a wave's split and its products do not overlap, so each is covered only by the
+// other waves of its SIMD (three or four).  The K loop loads whole steps without bounds checks (rows past the end
+// repeat the last row, the short last step is peeled off), K-contiguous operands 16 bytes at a time whatever the
+// rows' alignment, M/N-contiguous ones one value per K with the lanes along the row, and stages unpadded
+// XOR-swizzled rows; the epilogue branches once per block and stores through a uniform base plus a lane offset, of
+// 32 bits unless the rows lie too far apart (2000 x 2048 over 2048, rows of A 2^22 values apart: 100 us).  Measured against the same tiles with
 // checked loads, padded rows and an epilogue with per-element branches and addresses, batch 2, bit-identical:
 // 24576 x 512 x 123 with bias and ELU 90.5 -> 63.8 us, 24576 x 256 x 512 with bias and ELU 99.3 -> 82.0 us, 24576 x
 // 512 x 256 with the ELU gradient 116.6 -> 97.5 us, 4096 x 512 x 2048 127 -> 103 us, 1024 x 1024 x 256 15.6 -> 11.2
@@ -146,8 +148,9 @@ struct SplitLoader {
     }
 };
 
-// TM x TN output tile of WGM x WGN waves; MinWaves: the waves per SIMD the register allocation aims at (the 128
-// x 128 kernels fit 128 registers, so four waves, under a bound of 2 too, with better schedules: 99.4 -> 96.3 us).
+// TM x TN output tile of WGM x WGN waves; MinWaves: the waves per SIMD the register allocation aims at (under a
+// bound of 2 the 128 x 128 kernels still take 114 to 130 registers, so four waves, or three with an M-contiguous A
+// and a K-contiguous B, and have better schedules: 99.4 -> 96.3 us).
 // Offset: of a value in its tile, unsigned where that holds a tile's rows at their pitch.
 template <int TM, int TN, int WGM, int WGN, int Step, int MinWaves, class Offset, bool AK, bool BK>
 __global__ __launch_bounds__(WGM * WGN * kWave) __attribute__((amdgpu_waves_per_eu(MinWaves))) void split_kernel(

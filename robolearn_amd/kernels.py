@@ -86,13 +86,16 @@ def forward_split_count(m, n, k, batch, mode, kcontig=True):
     bf16 (heads, embedder input gradients, block input gradients): at least 256 workgroups.  Products
     the eight-wave kernel takes (both operands K-contiguous, m and n multiples of 256, K of 128) count
     its narrowest tiles, 256 x 64, which fill the GPU without partials or a reduction launch, and split
-    only in multiples of 128 of K; the others count 256x128 tiles, each split >= 128 of K.  A bf16 block
+    only in multiples of 128 of K; the others count 256x128 tiles, each split >= 128 of K.  Most of the others run on
+    64x64 tiles, which need no split (head forward 2 x 2048 x 101 over 512: 8.1 us whole, 12.1 us in the 4 splits
+    counted here; 4096 x 39 over 512 10.4 and 11.8 us), but another count adds in another order, which
+    whole updates amplify.  A bf16 block
     forward product is not split even where its tiles leave CUs idle (README shape): the split loses
     the BatchNorm moments of the epilogue and adds a reduction, which measured slower.
     fp32: 64x64 tiles, whose K loop is latency-bound when few workgroups share a CU; at least 1024
     workgroups, each split >= 256 of K: a split costs a reduction launch, which a shorter K loop
-    repays only past that (Cartpole input gradient 1024 x 1024 over K = 256: 17.8 us unsplit, 25.2 us
-    in two splits)."""
+    repays only past that (Cartpole input gradient, twin 1024 x 1024 over K = 256: 12.8 us unsplit,
+    23.7 us in two splits)."""
     splits = 1
     if mode == BF16:
         if kcontig and m % 256 == 0 and n % 256 == 0 and k % 128 == 0:
@@ -183,21 +186,21 @@ def split_count(m, n, k, batch, mode):
     """K splits for a weight-gradient product (small output, K = rows).
 
     bf16: at least two 256x128-tile workgroups per CU, each split >= 1024 of K; >= 128 of K
-    when the output does not tile by 256 (a narrow head or embedder: those products run on
-    the 256x128 kernel, whose workgroups are short enough that more of them pays: README head
-    dW 101 x 512 over 2048 rows 30.7 us in 8 splits, 22.6 in 16; embedder dW 256 x 31 over 4096
-    rows 24.0 us in 16, 17.5 in 32).  For the
-    256x256-tile kernel a longer split beats more workgroups: its partials cost a write and a
-    read of splits x M x N floats (README dW 2048 x 512 over 4096 rows: 44 us at 4 splits, 52 us
-    at 8).
-    fp32: the MFMA-issue-bound fp32 kernel runs 64x64 tiles for such products; at least 1024
-    workgroups (four per CU), each split >= 256 of K, whose reduction then costs less than the
-    shorter K loops save (Cartpole 256 x 1024 over 1024 rows: 23.6 us in 4 splits, 25.9 in 8); an
+    when the output does not tile by 256 (a narrow head or embedder, most of which run on 64x64
+    tiles: twin head dW 101 x 512 over 2048 rows 10.7 us in 8 splits, 12.2 in the 16 counted
+    here; 101 x 1024 over 8192 rows 24.7 us in 16, 28.4 in 32; embedder dW 256 x 31 over 4096
+    rows 9.5 us in 16, 8.8 in 32; the counts stay as they are, since others add in another
+    order).  For the 256x256-tile kernel a longer split beats more workgroups: its partials cost a
+    write and a read of splits x M x N floats (twin README dW 2048 x 512 over 4096 rows: 54 us in 2
+    splits, 44 in 4, 60 in 8).
+    fp32: 64x64 tiles for such products; at least 1024 workgroups (four per CU), each split >= 256
+    of K, whose reduction then costs less than the shorter K loops save (twin Cartpole 256 x 1024
+    over 1024 rows: 23.7 us in 2 splits, 22.6 in 4, 26.0 in 8); an
     output of at most 65,536 values (a head) takes splits down to 64 of K, since its reduction is
     nearly free.  Mode 2 outputs of more than 64 rows and columns whose splits reach 256 of the
     eight-wave 128x128-tile workgroups run there: at least 512 of them (two per CU), each split
-    >= 384 of K (PPO c3 dW 256 x 512 over 24576 rows: 105.7 us in 16 splits, 98.0 in 32; 128 x 256:
-    36.6 us in 64, 39.2 in 128)."""
+    >= 384 of K (twin PPO dW 256 x 512 over 24576 rows: 92.3 us in 16 splits, 88.2 in 32, 91.4 in
+    64; 128 x 256: 37.4 us in 32, 31.4 in 64, 33.8 in 128)."""
     splits = 1
     if mode == BF16:
         tiles = ((m + 255) // 256) * ((n + 127) // 128) * batch
@@ -355,9 +358,14 @@ def sample_indices(idx, *, seed, count=None, fixed_count=0, counter=None, stream
 
 def actor_act_fits(rows, obs_dim, hidden, blocks, action_dim) -> bool:
     """Whether actor_act takes these sizes and is the faster way to act on them: it streams the weights once per
-    16 rows into one CU (34 us a megabyte up to 16 rows per CU), the layers one launch each.  In us, one launch
-    against layers eager / on the GPU: hidden 128, one block, 135,000 weights 22 against 98 / 49; hidden 200, two
-    blocks, 660,000 weights 84 against 133 / 96; hidden 256, two blocks, 1,100,000 weights 134 against 133 / 107."""
+    16 rows into one CU (30 to 33 us a megabyte, up to 4096 rows at once), the layers one launch each.  In us, one
+    launch against the layers issued one by one / captured in a graph: obs 4, hidden 128, one block (132,000 weights),
+    64 rows 22 against 98 / 43; obs 60, hidden 200, two blocks (660,000), 64 rows 85 against 140 / 90, 4096 rows 87
+    against 137 / 122; obs 123, hidden 256, two blocks (1,100,000), 64 rows 137 against 155 / 102.  The line is
+    drawn for calls made one by one: a captured graph of the layers is the faster way at the widest networks below it
+    (obs 123, hidden 256, one block, 64 rows: 70 against 115 / 63).  Past 4096 rows a second round of workgroups doubles
+    the launch's time: small networks would still gain (hidden 64, two blocks, 8192 rows 33 against 152 / 68), those
+    near the weight limit lose (hidden 256, one block, 8192 rows 140 against 118 / 113)."""
     weights = hidden * (obs_dim + 8 * hidden * blocks + 2 * action_dim)
     return (hidden <= 256 and blocks <= 8 and obs_dim <= 1024 and 2 * action_dim <= 256 and rows <= 4096
             and weights <= 700_000)
