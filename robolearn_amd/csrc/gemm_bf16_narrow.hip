@@ -261,20 +261,25 @@ void launch(const Params& p, hipStream_t stream) {
 }  // namespace narrow
 
 // One round of 256 x 128 tiles (512: two workgroups per CU, however few of them the last round fills) takes about as
-// long as 1500 of the small ones, whose operand reuse is four times smaller, or as 1800 where an operand is M- or
-// N-contiguous and the large tiles transpose it; the additions to K are what a tile costs before and after its K loop.
-// The line is fitted to 1516 random products of 128 large tiles and more (24 to 20000 rows and columns, K from 24 to
-// 16000, all layouts, whole and split).  Of the 679 that it gives the small tiles 35 are 3 to 15 % slower there and the
-// others up to 3.9 times faster; of the 837 that it leaves to the large tiles 429 would take up to 2.2 times as long on
-// small ones and 244 would be 5 to 60 % faster.  With fewer large tiles the small ones always won (1.18 to 5.8 times
-// faster).  500 x 16000 over 1000, twin: 100 us on small tiles, 64 on large ones; 16400 x 400 over 8200 421 and 335 us;
-// 16384 x 1024 over 160, twin 43 and 46 us; 4096 x 512 over 160, twin 10.1 and 17.6 us.
+// long as `tiles` of the small ones, whose operand reuse is four times smaller; wide_fixed and kNarrowFixed are what a
+// tile costs before and after its K loop, in K.
+// The lines are fitted to 3416 products of 128 large tiles and more: 1957 random ones (24 to 20000 rows and columns, K
+// from 24 to 16000, all layouts, whole and split) and 1459 heads, embedders and gradients of theirs (256 to 32768 rows).
+// Of the 1976 that take the small tiles 74 are 3 to 16 % slower there and the others up to 4.5 times faster; of the 1440
+// that take the large ones 857 would take up to 2.5 times as long on small ones and 338 would be 5 to 49 % faster.  With
+// fewer large tiles the small ones always won (1.18 to 5.8 times faster).  Small against large tiles, twin products: 500
+// x 16000 over 1000 100 and 64 us; 8192 x 101 over 1024 in four splits 27 and 40 us; 16384 x 1024 over 160 52 and 54 us;
+// 4096 x 512 over 160 10 and 18 us; one member, 16400 x 400 over 8200 421 and 335 us.
 // Operands that do not load 16 bytes at a time, which the large tiles read one value at a time, take the small tiles at
 // any size: 1.07 to 26 times faster, 3.2 times in the middle, in 1443 random products (3190 x 4972 over 29 is 13 %
 // slower); 2396 x 567 over 12951 in four splits, twin: 214 against 919 us.
-constexpr int kRowTilesPerRound = 1500, kTransposedTilesPerRound = 1800;
-constexpr int kWideRound = 512;
-constexpr int kNarrowFixed = 128, kWideFixed = 256;
+struct Round {
+    int tiles, wide_fixed;
+};
+constexpr Round kRows{1500, 500};            // both operands K-contiguous
+constexpr Round kTransposed{1900, 320};      // an operand that the large tiles transpose
+constexpr Round kScalarOutput{1900, 1000};   // output rows that both store one value at a time
+constexpr int kWideRound = 512, kNarrowFixed = 192;
 
 bool narrow_eligible(const Params& p, int a_bf16, int b_bf16, bool ak, bool bk) {
     const long long products = static_cast<long long>(p.batch) * p.splits;
@@ -285,8 +290,8 @@ bool narrow_eligible(const Params& p, int a_bf16, int b_bf16, bool ak, bool bk) 
     const long long tiles = rows * ceil_div(p.n, narrow::kTileEdge) * products;
     const long long wide = static_cast<long long>(ceil_div(p.m, 256)) * ceil_div(p.n, 128) * products;
     const long long rounds = (wide + kWideRound - 1) / kWideRound;
-    const long long per_round = ak && bk ? kRowTilesPerRound : kTransposedTilesPerRound;
-    return tiles * (p.k_per_split + kNarrowFixed) < per_round * rounds * (p.k_per_split + kWideFixed);
+    const Round& round = !p.out_vec ? kScalarOutput : ak && bk ? kRows : kTransposed;
+    return tiles * (p.k_per_split + kNarrowFixed) < rounds * round.tiles * (p.k_per_split + round.wide_fixed);
 }
 
 void launch_narrow(const Params& p, bool ak, bool bk, hipStream_t stream) {

@@ -84,6 +84,7 @@ void* create_plan(int m, int n, int k, int transa, int transb, int lda, int ldb,
     const int operand_bytes = plan->operands_16bit ? 2 : 4;
     p.a_vec = p.lda * operand_bytes % 16 == 0;
     p.b_vec = p.ldb * operand_bytes % 16 == 0;
+    p.out_vec = p.n % 4 == 0 && (p.splits > 1 || p.ldd % 4 == 0);
     const char* kernel = rl::gemm::kernel_name(plan->mode, p, plan->operands_16bit, plan->operands_16bit,
                                                transb == 0, transa == 1);
     const char* precision = plan->mode == 0 ? "fp32" : (plan->mode == 3 ? "fp16" : "bf16");

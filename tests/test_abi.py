@@ -94,7 +94,7 @@ def test_dense_plan_metadata_names_the_kernel(rows, cols, k, input_dtype, kernel
     assert plan_kernel(rows, cols, k, input_dtype) == kernel
 
 
-# either side of the line in rows, K, rounds of large tiles and 16-byte rows of the operands; (500, 16000, 1000) takes 64 us
+# either side of the line in rows, K, rounds of large tiles and 16-byte rows of operands and output; (500, 16000, 1000) takes 64 us
 # on the 256 x 128 tiles and 100 us on the 64 x 64 ones as a twin product
 @pytest.mark.parametrize("rows,cols,k,transa,transb,kernel", [
     (500, 16000, 1000, 1, 0, "mfma_256x128"),
@@ -108,6 +108,8 @@ def test_dense_plan_metadata_names_the_kernel(rows, cols, k, input_dtype, kernel
     (3000, 3000, 40, 1, 0, "mfma_64x64"),
     (16400, 16400, 264, 0, 1, "mfma_256x128"),
     (24, 16000, 1000, 1, 0, "mfma_64x64"),
+    (65536, 101, 1024, 1, 0, "mfma_64x64"),
+    (65536, 104, 1024, 1, 0, "mfma_256x128"),
 ])
 def test_bf16_products_take_the_faster_tiles(rows, cols, k, transa, transb, kernel):
     assert plan_kernel(rows, cols, k, 3, transa, transb) == kernel
