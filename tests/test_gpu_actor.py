@@ -97,3 +97,11 @@ def test_refused_observations_draw_no_noise(gpu):
     with pytest.raises(ValueError):
         K.actor_act(rows, agent._act_parameters, None, torch.empty(4, 2, device=gpu), obs_dim=3, hidden=32, blocks=1,
                     action_dim=2)
+
+
+# the largest observations, action counts and block counts of the launch, and either side of its two instances
+@pytest.mark.parametrize("obs_dim,action_dim,hidden,blocks", [(1024, 80, 256, 0), (1024, 2, 128, 1), (48, 5, 64, 8),
+                                                              (512, 64, 128, 1), (513, 64, 128, 1), (9, 3, 129, 2)])
+@pytest.mark.parametrize("rows", [1, 33])
+def test_one_launch_actor_at_its_limits(gpu, obs_dim, action_dim, hidden, blocks, rows):
+    test_one_launch_actor_matches_float64(gpu, obs_dim, action_dim, hidden, blocks, rows)
