@@ -63,3 +63,27 @@ def test_narrow_products(gpu, m, n, k, splits, batch, pad, a_kcontig, b_kcontig)
                                                 (1016, 4216, 1416, 1, 2), (1001, 8101, 552, 1, 2)])
 def test_products_at_the_line_between_tiles(gpu, m, n, k, splits, batch, pad, a_kcontig, b_kcontig):
     test_narrow_products(gpu, m, n, k, splits, batch, pad, a_kcontig, b_kcontig)
+
+
+# rows too far apart for the small tiles' offsets run the 256 x 128 tiles, rows of 16 bytes (2^22) and others alike
+@pytest.mark.parametrize("a_kcontig,b_kcontig", [(True, True), (True, False), (False, True), (False, False)])
+@pytest.mark.parametrize("pitch", [(1 << 22) - 1, 1 << 22, (1 << 22) + 1])
+@pytest.mark.parametrize("far", [0, 1])
+def test_far_rows_give_the_same_bits(gpu, far, pitch, a_kcontig, b_kcontig):
+    print(f"case far bf16 operand={far} pitch={pitch} ak={a_kcontig} bk={b_kcontig}", flush=True)
+    m, n, k = 70, 133, 41
+    g = torch.Generator(device=gpu).manual_seed(pitch)
+    shapes = ((m, k) if a_kcontig else (k, m), (n, k) if b_kcontig else (k, n))
+    values = [torch.randn(s, generator=g, device=gpu).bfloat16() for s in shapes]
+    results = []
+    for apart in (False, True):
+        ops = list(values)
+        if apart:
+            rows, cols = shapes[far]
+            store = torch.empty((rows - 1) * pitch + cols, dtype=torch.bfloat16, device=gpu)
+            ops[far] = store.as_strided((rows, cols), (pitch, 1)).copy_(values[far])
+        d = torch.full((m, n), 7.0, device=gpu)
+        K.gemm(ops[0], ops[1], d, m=m, n=n, k=k, a_kcontig=a_kcontig, b_kcontig=b_kcontig, lda=ops[0].stride(0),
+               ldb=ops[1].stride(0), ldd=n, mode=K.BF16)
+        results.append(d)
+    assert torch.equal(*results)
